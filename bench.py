@@ -435,7 +435,7 @@ def dom_name(c):
     cls = "%d,%d,%d,%d" % (c["la"], c["lb"], c["lc"], c["ld"])
     kind = c.get("kind", 0)
     if kind == 2:
-        return "k_generic (%s)" % cls
+        return "k_generic (%s)" % cls if c.get("alt") else "k_rows<%s>" % cls
     return "k_jk<%s,%s,%s>" % ("float" if kind >= 3 else "double", cls, "OS" if kind in (0, 3) else "Rys")
 
 

@@ -128,7 +128,7 @@ int pk_fock_jk(pk_ctx *ctx, const double *P, double *J, double *K, int memkind);
 int pk_fock_2e(pk_ctx *ctx, const double *P, double *G, int memkind);
 /* UHF: Jt = J[Pa + Pb], Ka = K[Pa], Kb = K[Pb]; G_a = Jt - Ka, G_b = Jt - Kb
  * (_compute_2e_fock_uhf, base.h:75-93).  One build (FP64): the Obara-Saika
- * and cooperative classes compute each quartet once and digest it into J of
+ * and row-kernel classes compute each quartet once and digest it into J of
  * Pa + Pb and both exchange matrices; the per-lane Rys classes run once per
  * spin density.  Host or device pointers; Jt, Ka or Kb may be NULL.  Packed
  * arrays for batches, as pk_fock_jk.  Runs eagerly (no graph). */
@@ -187,7 +187,7 @@ typedef struct pk_class_stats {
                                      integrals for an FP32 list, or the cooperative kernel for a
                                      class with per-lane Rys kernels */
     int32_t kind;                 /* kernels that run the list: 0 per-lane Obara-Saika (FP64),
-                                     1 per-lane Rys (FP64), 2 cooperative (FP64), 3 per-lane
+                                     1 per-lane Rys (FP64), 2 row or cooperative kernel (FP64), 3 per-lane
                                      Obara-Saika (FP32), 4 per-lane Rys (FP32) */
 } pk_class_stats;
 int pk_ctx_profile(pk_ctx *ctx, int enable);

@@ -73,20 +73,11 @@ namespace pk {
 // Contracted Rys accumulators per lane: a class whose NE x NCD intermediates
 // exceed the budget runs in chunks of ket components, each chunk recomputing
 // the roots and 2-D integrals.  Measured per class on n-C10H22 / cc-pVTZ,
-// budget 64 against 48: 0.56-0.88x the time for the chunked d/f classes (fewer
-// chunks), and (fp|dp) gains a per-lane kernel (9 chunks; 0.63x the
-// cooperative kernel's time); budget 80 against 64: 0.83-0.94x for most chunked
-// classes ((fp|ps) 4.9 -> 3.7 ms, (fp|pp) 5.1 -> 4.2 ms, (fp|dp) 7.0 -> 6.2 ms).
+// budget 80 against 64: 0.83-0.94x for most chunked classes ((fp|ps) 4.9 -> 3.7 ms).
 #ifndef PK_ACC_BUDGET
 #define PK_ACC_BUDGET 80
 #endif
 constexpr int kAccBudget = PK_ACC_BUDGET;
-constexpr int kMaxChunks = 12;  // larger classes run in the cooperative kernel
-// Which f classes get per-lane kernels is decided at this budget: at 80,
-// (fp|dd) and (fp|fp) would fit 12 and 10 chunks, but (fp|fp) is slower so
-// (2.0 -> 2.7 ms) and the two triple the kernel shards' build time.
-constexpr int kTmplBudget = 64;
-
 #ifndef PK_ACC_BUDGET32
 #define PK_ACC_BUDGET32 128
 #endif
@@ -105,12 +96,21 @@ constexpr int chunk_size(int la, int lb, int lc, int ld, int budget = kAccBudget
     return (ncd + nch - 1) / nch;
 }
 
-// classes with a per-lane Rys kernel: every s/p/d class, and f classes of at
-// most kMaxChunks ket-component chunks (the rest run in the cooperative kernel)
-constexpr bool rys_tmpl_available(int la, int lb, int lc, int ld) {
-    const int ncd = ncart(lc) * ncart(ld), ch = chunk_size(la, lb, lc, ld, kTmplBudget);
-    return la <= 2 || (ncd + ch - 1) / ch <= kMaxChunks;
+// Classes with a row kernel (eri_rows.h) instead of a per-lane Rys kernel: kets
+// of at least nine components, and (ds) kets under (fd| and (ff| bras.  Measured
+// on n-C10H22 / cc-pVTZ (ms, per-lane or one-quartet-per-wave kernel -> rows):
+// (fd|dp) 8.1 -> 2.1, (fp|dp) 6.2 -> 2.4, (dp|dp) 8.1 -> 3.4, (dd|dp) 7.3 -> 3.4,
+// (fd|pp) 5.4 -> 1.7, (dp|pp) 8.2 -> 4.8, (pp|pp) 4.4 -> 2.9, (fs|fs) 1.19 -> 0.96,
+// (fd|ds) 4.1 -> 3.1, (ff|ds) 1.5 -> 1.1.  Below nine components a row is too
+// short for its share of the roots and 2-D integrals: (dp|ps) 7.7 -> 15.7,
+// (dd|ps) 4.7 -> 5.2, (fp|ds) 3.5 -> 4.2, (dd|ds) 3.8 -> 3.9.
+constexpr bool rows_class(int la, int lb, int lc, int ld) {
+    if (lc + ld < 2 || (la == 2 && lb == 0)) return false;  // (ds| bras: Obara-Saika classes
+    if (lc == 2 && ld == 0) return la == 3 && lb >= 2;
+    return true;
 }
+// classes with a per-lane Rys kernel
+constexpr bool rys_tmpl_available(int la, int lb, int lc, int ld) { return !rows_class(la, lb, lc, ld); }
 
 // classes with an Obara-Saika kernel: L <= 4 and [e0|f0] accumulators <= 54
 constexpr bool os_available(int la, int lb, int lc, int ld) {

@@ -55,6 +55,7 @@ struct JKArgs {
     int nseg;
     int kcols;
     int segmode;
+    int chunk;  // row kernels: groups of quartets per turn of a wave (see eri_rows.h)
 };
 
 // Wave handled by this wave slot.  With remap, workgroup b (dispatched to XCD

@@ -1,9 +1,9 @@
 // pk_fock.hip — host side of the MI355X Fock-build engine and its C ABI
 // (include/pk_fock.h).  Per-lane class kernels live in eri_kernels.h (instantiated
-// in pk_kernels.hip), the cooperative kernel for large f classes and for ERI
-// output in eri_generic.h; this file builds the shell pairs, the Schwarz table
-// and the screened quartet work lists, and launches the kernels on the
-// context's stream.
+// in pk_kernels.hip), the row kernels of the large classes in eri_rows.h, the
+// cooperative kernel for ERI output in eri_generic.h; this file builds the shell
+// pairs, the Schwarz table and the screened quartet work lists, and launches the
+// kernels on the context's stream.
 //
 // Reference path replaced: src/integrals/base.h:57-93 (_compute_2e_fock[_uhf]),
 // src/integrals/os.cpp:1435-1625 and rys.cpp:701-824 (the Fock builds),
@@ -28,6 +28,7 @@
 #include "eri_classes.h"
 #include "eri_generic.h"
 #include "eri_grad.h"
+#include "rows_table.h"
 
 // per-class launchers, defined in pk_kernels.hip
 #define PK_DECL(a, b, c, d, shard)                                                             \
@@ -68,6 +69,11 @@ constexpr int64_t kSideMinQuartets = 1 << 20;
 // Segment mode of the per-lane kernels (see k_jk): at most kSegWaves waves of
 // one bra per segment, and at most kSegLdsMax bytes of LDS exchange rows.
 constexpr int kSegWaves = 16;
+// Row kernels: a list is cut into about kRowItems work items (workgroups) of at
+// most kRowKetsMax kets; measured on n-C10H22 / cc-pVTZ, 8192 items: the same or
+// up to 1.6x slower (a workgroup flushes its exchange rows once).
+constexpr size_t kRowItems = 4096, kRowKetsMax = 1024;
+constexpr size_t kLdsMax = 160 * 1024;  // LDS of a CU, and of one workgroup
 // primitive quartets per shell quartet below which a list of a pk::seg_alt_class
 // runs in segment mode (6-31G* water clusters: 11-13; cc-pVTZ alkanes: 40-80)
 constexpr double kSegAltPrim = 24.0;
@@ -83,7 +89,7 @@ constexpr int kQuartClasses = kPairClasses * (kPairClasses + 1) / 2;
 struct ClassFns {
     int la, lb, lc, ld;
     bool has_os;    // Obara-Saika per-lane kernel
-    bool has_tmpl;  // Rys per-lane kernel (else the cooperative kernel)
+    bool has_tmpl;  // Rys per-lane kernel (else the row kernel, pk::rows_class)
     bool seg;       // the per-lane kernels run in segment mode (pk::seg_class)
     bool seg_alt;   // the OS kernel also exists in segment mode (pk::seg_alt_class)
     void (*jk_os)(const pk::JKArgs &, int, int, hipStream_t, int &);
@@ -107,6 +113,23 @@ struct ClassFns {
 // pair classes (0,0) (1,0) (1,1) (2,0) (2,1) (2,2) (3,0) (3,1) (3,2) (3,3).
 const ClassFns kClasses[kQuartClasses] = {PK_FOR_EACH_CLASS(PK_ENTRY)};
 #undef PK_ENTRY
+
+// row kernels by quartet class
+const pk::RowsEntry *rows_table() {
+    static const std::vector<pk::RowsEntry> t = [] {
+        std::vector<pk::RowsEntry> v(kQuartClasses);
+        pk_rows_register<0>(v.data());
+        pk_rows_register<1>(v.data());
+        pk_rows_register<2>(v.data());
+        pk_rows_register<3>(v.data());
+        pk_rows_register<4>(v.data());
+        pk_rows_register<5>(v.data());
+        pk_rows_register<6>(v.data());
+        pk_rows_register<7>(v.data());
+        return v;
+    }();
+    return t.data();
+}
 
 int quart_class(int cb, int ck) { return cb * (cb + 1) / 2 + ck; }
 int class_la(int c) {
@@ -218,6 +241,7 @@ struct ClassWork {
     int nseg = 0;          // segments: runs of at most kSegWaves waves of one bra
     int *d_seg = nullptr;  // [nseg + 1] first wave of each segment
     int kcols = 0;         // LDS columns of an exchange row (largest molecule)
+    int group = 0;         // row kernels: most kets of a work item
     int kernels = 0;
     double ms_total = 0.0;
     int64_t builds = 0;
@@ -313,7 +337,7 @@ namespace {
 bool use_os(const pk_ctx *c, const ClassFns &f) { return f.has_os && c->engine != PK_ENGINE_RYS; }
 
 // Kernels that run a class list (pk_class_stats.kind): 0 / 3 per-lane OS in
-// FP64 / FP32, 1 / 4 per-lane Rys in FP64 / FP32, 2 cooperative (FP64).
+// FP64 / FP32, 1 / 4 per-lane Rys in FP64 / FP32, 2 row or cooperative kernel (FP64).
 int list_kind(const pk_ctx *c, const ClassWork &w) {
     const ClassFns &f = kClasses[w.cls];
     const bool fp32 = w.prec == PK_PREC_MIXED && !w.alt;
@@ -348,58 +372,12 @@ void free_work(pk_ctx *c) {
 // all of class (cb, ck) with cb >= ck.  out gets NA NB NC ND values per quartet.
 // One 64-lane workgroup per item; the dynamic LDS holds the transferred 1-D
 // factors and the quartet's accumulators (at most 123 KB for (ff|ff)).
-// Cooperative kernels with the class fixed at compile time, for the J/K lists
-// of the classes without a per-lane kernel (null elsewhere), with
-// pk::gen_waves(class) waves per quartet.
-struct GenKernels {
-    const void *k1, *k2;  // one and two exchange densities
-    int waves;
-};
-template <int A, int B, int C, int D>
-constexpr GenKernels gen_kernels() {
-    if constexpr (!pk::rys_tmpl_available(A, B, C, D)) {
-        constexpr int W = pk::gen_waves(A, B, C, D);
-        return GenKernels{(const void *)pk::k_generic<1, A, B, C, D, W>, (const void *)pk::k_generic<2, A, B, C, D, W>, W};
-    } else {
-        return GenKernels{nullptr, nullptr, 1};
-    }
-}
-#define PK_GEN_ENTRY(a, b, c, d, shard) gen_kernels<a, b, c, d>(),
-const GenKernels kGenKernels[kQuartClasses] = {PK_FOR_EACH_CLASS(PK_GEN_ENTRY)};
-
 int launch_generic(const pk::GenArgs &a, hipStream_t s) {
     if (a.nitems <= 0) return PK_OK;
-    if (!a.eri_mode) {
-        const int cb = pk::pair_class(a.la, a.lb), ck = pk::pair_class(a.lc, a.ld);
-        const GenKernels &g = kGenKernels[quart_class(cb, ck)];
-        const void *k = a.B2 ? g.k2 : g.k1;
-        if (k) {
-            static std::atomic<int> attr_done[2 * kQuartClasses];  // zero-initialised
-            const size_t bytes = pk::generic_lds_bytes(a.la, a.lb, a.lc, a.ld, 64 * g.waves);
-            std::atomic<int> &done = attr_done[2 * quart_class(cb, ck) + (a.B2 ? 1 : 0)];
-            if (!done.load()) {
-                PK_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)pk::generic_lds_bytes(kMaxL, kMaxL, kMaxL, kMaxL)));
-                done.store(1);
-            }
-            pk::GenArgs x = a;
-            void *args[] = {&x};
-            PK_HIP(hipLaunchKernel(k, dim3(a.nitems), dim3(64 * g.waves), args, bytes, s));
-            return PK_OK;
-        }
-    }
-    static const size_t max_bytes = pk::generic_lds_bytes(kMaxL, kMaxL, kMaxL, kMaxL);
-    static const hipError_t attr1 =
-        hipFuncSetAttribute((const void *)pk::k_generic<1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_bytes);
-    static const hipError_t attr2 =
-        hipFuncSetAttribute((const void *)pk::k_generic<2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_bytes);
-    PK_HIP(attr1);
-    PK_HIP(attr2);
-    const size_t bytes = pk::generic_lds_bytes(a.la, a.lb, a.lc, a.ld);
-    if (a.B2)
-        hipLaunchKernelGGL(pk::k_generic<2>, dim3(a.nitems), dim3(64), bytes, s, a);
-    else
-        hipLaunchKernelGGL(pk::k_generic<1>, dim3(a.nitems), dim3(64), bytes, s, a);
+    static const hipError_t attr = hipFuncSetAttribute((const void *)pk::k_generic, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                       (int)pk::generic_lds_bytes(kMaxL, kMaxL, kMaxL, kMaxL));
+    PK_HIP(attr);
+    hipLaunchKernelGGL(pk::k_generic, dim3(a.nitems), dim3(64), pk::generic_lds_bytes(a.la, a.lb, a.lc, a.ld), s, a);
     PK_HIP(hipGetLastError());
     return PK_OK;
 }
@@ -498,7 +476,7 @@ void parallel_for(size_t n, F f) {
 // primitive count and shells, cut into waves of at most 64 kets; the waves of all
 // molecules form one list per class.  In mixed precision the kets with
 // qmax_bra * qmax_ket < cutoff form a second, FP32 list of the class (classes
-// of the cooperative kernel stay FP64).
+// of the row kernels stay FP64).
 int ensure_side(pk_ctx *c);
 
 int build_work(pk_ctx *c) {
@@ -541,10 +519,11 @@ int build_work(pk_ctx *c) {
         for (int ck = 0; ck <= cb; ++ck) {
             const int cls = quart_class(cb, ck);
             const ClassFns &f = kClasses[cls];
-            const bool split = mixed && f.has_tmpl;
-            // kets per work item: a wave of 64 lanes for the per-lane kernels,
-            // a few quartets per workgroup for the cooperative kernel
-            const size_t group = f.has_tmpl ? 64 : 4;
+            const bool rows = !f.has_tmpl;
+            const bool split = mixed && !rows;
+            // kets per work item: a wave of 64 lanes for the per-lane kernels;
+            // for the row kernels a workgroup's share of a bra's kets (below)
+            size_t group = 64;
             // bra tasks of every molecule, in order
             std::vector<std::pair<int, int>> tasks;
             for (int m = 0; m < c->nmol; ++m)
@@ -577,6 +556,14 @@ int build_work(pk_ctx *c) {
                     o.k0 = prec == PK_PREC_FP64 ? 0 : n_hi;
                     o.k1 = std::max(o.k0, prec == PK_PREC_FP64 ? n_hi : n_tol);
                 });
+                if (rows) {
+                    // about kRowItems work items of equal ket counts, whole groups
+                    size_t tot = 0;
+                    for (const BraRange &o : outs) tot += o.k1 - o.k0;
+                    const size_t qw = rows_table()[cls].qw;
+                    group = std::min<size_t>(kRowKetsMax, std::max<size_t>(1, tot / kRowItems));
+                    group = (group + qw - 1) / qw * qw;
+                }
                 ClassWork w;
                 w.cls = cls;
                 w.prec = prec;
@@ -640,10 +627,26 @@ int build_work(pk_ctx *c) {
                 }
                 if (w.nquart == 0) continue;
                 w.nwaves = (int)nw;
+                if (rows) {
+                    // most expensive work items first, so that none of them ends the list
+                    // alone (n-C10H22 / cc-pVTZ: (dd|dp) 5.2 -> 3.4 ms, (fd|dp) 3.1 -> 2.1 ms)
+                    std::vector<double> cost(nw, 0.0);
+                    for (size_t i = 0; i < nw; ++i) {
+                        const int kb = c->pairs[packed[i]].nprim;
+                        for (int j = 0; j < packed[2 * nw + i]; ++j) cost[i] += 1.0 + kb * c->pairs[kets[packed[nw + i] + j]].nprim;
+                    }
+                    std::vector<int> o(nw);
+                    std::iota(o.begin(), o.end(), 0);
+                    std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+                    std::vector<int> q(4 * nw);
+                    for (int k = 0; k < 4; ++k)
+                        for (size_t i = 0; i < nw; ++i) q[k * nw + i] = packed[k * nw + o[i]];
+                    packed.swap(q);
+                }
                 int rc;
                 if ((rc = dev_upload(&w.d_wave, packed, c->stream)) != PK_OK) return rc;
                 if ((rc = dev_upload(&w.d_kets, kets.get(), koff.back(), c->stream)) != PK_OK) return rc;
-                if (f.has_tmpl) {
+                if (!rows) {
                     // segments of the per-lane kernels: each bra's waves in runs
                     // of at most kSegWaves; LDS columns: the two ket shell types
                     // of the largest molecule
@@ -659,6 +662,13 @@ int build_work(pk_ctx *c) {
                     seg.push_back((int)nw);
                     w.nseg = (int)seg.size() - 1;
                     if ((rc = dev_upload(&w.d_seg, seg, c->stream)) != PK_OK) return rc;
+                } else {
+                    // LDS columns of the row kernels: the ket's second shell type
+                    w.group = (int)group;
+                    for (size_t t = 0; t < tasks.size(); ++t) {
+                        const int *tb = &c->tblk[5 * tasks[t].first];
+                        if (woff[t + 1] > woff[t]) w.kcols = std::max(w.kcols, tb[f.ld + 1] - tb[f.ld]);
+                    }
                 }
                 c->st.quartets += w.nquart;
                 c->st.primitive_quartets += w.nprimq;
@@ -717,7 +727,7 @@ BuildBufs ctx_bufs(pk_ctx *c) { return BuildBufs{c->d_Pn, c->d_A, c->d_B, c->d_P
 // Enqueue the class kernels of one build (the density already scaled into
 // sb.Pn, the accumulators cleared); nl counts the launches.  With sb.B2 set
 // (one-pass UHF) every list runs FP64 two-density digestion: the per-lane OS
-// kernels where the class has them, else the cooperative kernel.
+// or row kernels where the class has them, else the per-lane Rys kernels twice.
 int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipStream_t s, int &nl);
 
 // Side streams and events of a context, created on first use.
@@ -751,12 +761,12 @@ int launch_classes(pk_ctx *c, const BuildBufs &sb, bool events, int &nl) {
         // cost of a list: its measured time when the context has one (the first
         // large build of a context times every list, one at a time), else the
         // model flops over a typical rate of its kernel (TFLOP/s: per-lane OS
-        // ~10, per-lane Rys ~3, cooperative ~1.5)
+        // ~10, per-lane Rys ~3, row kernels ~6)
         std::vector<double> cost(c->work.size());
         for (size_t i = 0; i < cost.size(); ++i) {
             const ClassWork &w = c->work[i];
-            const int kind = list_kind(c, w) % 3;  // 0 OS, 1 Rys, 2 cooperative
-            cost[i] = w.cost_ms > 0.0 ? w.cost_ms : w.flops * 1e-9 / (kind == 0 ? 10.0 : kind == 1 ? 3.0 : 1.5);
+            const int kind = list_kind(c, w) % 3;  // 0 OS, 1 Rys, 2 rows
+            cost[i] = w.cost_ms > 0.0 ? w.cost_ms : w.flops * 1e-9 / (kind == 0 ? 10.0 : kind == 1 ? 3.0 : 6.0);
         }
         std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return cost[x] > cost[y]; });
         double load[kSideQueues + 1] = {};
@@ -823,6 +833,38 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
         // compiled both ways take it for lists of few primitive quartets per
         // shell quartet (atomic-bound), the plain kernel otherwise
         const bool seg_alt = f.seg_alt && use_os(c, f) && (double)w.nprimq <= c->seg_alt_prim * (double)w.nquart;
+        if (!f.has_tmpl) {
+            const pk::RowsEntry &r = rows_table()[w.cls];
+            const int rk = uhf ? 2 : 1;
+            const size_t wave_bytes = r.wave_bytes[rk - 1];
+            const void *k = uhf ? r.k2 : r.k1;
+            // exchange rows of the kets' second shells in LDS, beside at least one
+            // wave; then as many waves as fit, four (two workgroups per CU) at most
+            const size_t jrow = (size_t)pk::ncart(f.la) * pk::ncart(f.lb) * sizeof(double);
+            size_t krow = (size_t)rk * (pk::ncart(f.la) + pk::ncart(f.lb)) * w.kcols * sizeof(double) + jrow;
+            a.segmode = c->seg_on && krow + wave_bytes <= kLdsMax;
+            if (!a.segmode) krow = jrow;
+            int waves = w.block > 0 ? w.block / 64 : kDefaultBlock / 64;
+            const int groups = (w.group + r.qw - 1) / r.qw;  // of the largest work item
+            while (waves > 1 && (waves / 2 >= groups || krow + (size_t)waves * wave_bytes > kLdsMax)) waves /= 2;
+            // eight groups per turn of a wave, fewer where the item has fewer
+            a.chunk = std::max(1, std::min(8, groups / (2 * waves)));
+            w.block_run = 64 * waves;
+            static std::atomic<int> attr_done[2 * kQuartClasses];  // zero-initialised
+            std::atomic<int> &done = attr_done[2 * w.cls + rk - 1];
+            if (!done.load()) {
+                PK_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax));
+                done.store(1);
+            }
+            int grid = w.nwaves;
+            if (w.remap) grid = (grid + 7) / 8 * 8;
+            void *args[] = {&a};
+            PK_HIP(hipLaunchKernel(k, dim3(grid, r.rc), dim3(64 * waves), args, krow + (size_t)waves * wave_bytes, s));
+            w.kernels = 1;
+            ++nl;
+            if (events) PK_HIP(hipEventRecord(w.e1, s));
+            return PK_OK;
+        }
         const int nk = uhf && use_os(c, f) ? 2 : 1;
         {
             const size_t rows = (size_t)nk * (pk::ncart(f.la) + pk::ncart(f.lb)) * w.kcols +
@@ -847,7 +889,7 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
         if (w.remap) grid = (grid + 7) / 8 * 8;
         if (uhf && use_os(c, f)) {
             (alt ? f.jk_os_uhf_seg : f.jk_os_uhf)(a, grid, block, s, nl);
-        } else if (uhf && f.has_tmpl) {
+        } else if (uhf) {
             // per-lane Rys kernels once per spin density: J of each into A
             // (summing to J of Pa + Pb), exchange into B and B2
             pk::JKArgs x = a;
@@ -856,18 +898,15 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
             x.P = sb.PKb;
             x.B = sb.B2;
             f.jk_rys(x, grid, block, s, nl);
-        } else if (uhf) {
-            // handled by the cooperative kernel below
         } else if (use_os(c, f)) {
             if (alt)
                 (fp32 ? f.jk_os32_seg : f.jk_os_seg)(a, grid, block, s, nl);
             else
                 (fp32 ? f.jk_os32 : f.jk_os)(a, grid, block, s, nl);
-        } else if (f.has_tmpl && !(w.alt && w.prec == PK_PREC_FP64)) {
+        } else if (!(w.alt && w.prec == PK_PREC_FP64)) {
             (fp32 ? f.jk_rys32 : f.jk_rys)(a, grid, block, s, nl);
         }
-        if ((uhf && !use_os(c, f) && !f.has_tmpl) ||
-            (!uhf && !use_os(c, f) && !(f.has_tmpl && !(w.alt && w.prec == PK_PREC_FP64)))) {
+        if (!uhf && !use_os(c, f) && w.alt && w.prec == PK_PREC_FP64) {
             pk::GenArgs g{};
             g.wave_bra = a.wave_bra;
             g.wave_start = a.wave_start;
@@ -880,12 +919,9 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
             g.prims = a.prims;
             g.hz = a.hz;
             g.P = a.P;
-            g.PK = uhf ? a.PK : a.P;
-            g.PK2 = a.PK2;
             g.Q = a.Q;
             g.A = a.A;
             g.B = a.B;
-            g.B2 = a.B2;
             g.tol = a.tol;
             g.nitems = w.nwaves;
             g.la = f.la;
