@@ -28,6 +28,7 @@
 #include "eri_classes.h"
 #include "eri_generic.h"
 #include "eri_grad.h"
+#include "grad_table.h"
 #include "rows_table.h"
 
 // per-class launchers, defined in pk_kernels.hip
@@ -73,6 +74,7 @@ constexpr int kSegWaves = 16;
 // most kRowKetsMax kets; measured on n-C10H22 / cc-pVTZ, 8192 items: the same or
 // up to 1.6x slower (a workgroup flushes its exchange rows once).
 constexpr size_t kRowItems = 4096, kRowKetsMax = 1024;
+constexpr size_t kGradItems = 8192;  // gradient work items (one wave each) of a class, about
 constexpr size_t kLdsMax = 160 * 1024;  // LDS of a CU, and of one workgroup
 // primitive quartets per shell quartet below which a list of a pk::seg_alt_class
 // runs in segment mode (6-31G* water clusters: 11-13; cc-pVTZ alkanes: 40-80)
@@ -126,6 +128,24 @@ const pk::RowsEntry *rows_table() {
         pk_rows_register<5>(v.data());
         pk_rows_register<6>(v.data());
         pk_rows_register<7>(v.data());
+        return v;
+    }();
+    return t.data();
+}
+
+// gradient kernels by ordered class (bra pair class, ket pair class)
+static_assert(PK_GRAD_PAIRS == kPairClasses, "gradient kernels cover every pair class");
+const pk::GradEntry *grad_table() {
+    static const std::vector<pk::GradEntry> t = [] {
+        std::vector<pk::GradEntry> v(PK_GRAD_PAIRS * PK_GRAD_PAIRS);
+        pk_grad_register<0>(v.data());
+        pk_grad_register<1>(v.data());
+        pk_grad_register<2>(v.data());
+        pk_grad_register<3>(v.data());
+        pk_grad_register<4>(v.data());
+        pk_grad_register<5>(v.data());
+        pk_grad_register<6>(v.data());
+        pk_grad_register<7>(v.data());
         return v;
     }();
     return t.data();
@@ -249,6 +269,15 @@ struct ClassWork {
     hipEvent_t e0 = nullptr, e1 = nullptr;
 };
 
+// Gradient work of one ordered class: items (bra, first ket, kets, bra primitives)
+// into the context's gradient order.
+struct GradWork {
+    int cls = 0;  // bra class * kPairClasses + ket class
+    int nitems = 0;
+    double cost = 0.0;
+    int *d_items = nullptr;  // [4][nitems]
+};
+
 template <typename T>
 int dev_upload(T **dst, const T *src, size_t n, hipStream_t s) {
     *dst = nullptr;
@@ -309,6 +338,9 @@ struct pk_ctx {
     int *d_pair_sh = nullptr;
     std::vector<ClassWork> work;
     bool work_ok = false;
+    std::vector<GradWork> gwork;  // gradient work items, built by the first gradient at a tolerance
+    int *d_gorder = nullptr;
+    double gwork_tol = -1.0;
     int engine = PK_ENGINE_OS;
     double tol = 1e-10;
     int precision = PK_PREC_FP64;
@@ -352,6 +384,15 @@ void drop_graph(pk_ctx *c) {
     c->gexec = nullptr;
     c->graph = nullptr;
     c->graph_ok = false;
+}
+
+void free_grad(pk_ctx *c) {
+    for (GradWork &w : c->gwork)
+        if (w.d_items) (void)hipFree(w.d_items);
+    c->gwork.clear();
+    if (c->d_gorder) (void)hipFree(c->d_gorder);
+    c->d_gorder = nullptr;
+    c->gwork_tol = -1.0;
 }
 
 void free_work(pk_ctx *c) {
@@ -692,6 +733,116 @@ int build_work(pk_ctx *c) {
         if ((rc = ensure_side(c)) != PK_OK) return rc;
     }
     c->work_ok = true;
+    return PK_OK;
+}
+
+// Work items of the gradient (one molecule): for every ordered pair of pair
+// classes and every bra, all kets with qmax_bra qmax_ket >= tol.  The pairs of a
+// class are ordered by ordering group, then Schwarz bound, so the kets of a bra
+// are one range per group (neighbouring ranges joined) and no list per bra is
+// needed.
+int build_grad(pk_ctx *c) {
+    if (c->gwork_tol == c->tol) return PK_OK;
+    free_grad(c);
+    const int np = (int)c->pairs.size();
+    std::vector<int> order;
+    std::vector<int> cbeg(kPairClasses + 1, 0);
+    std::vector<std::vector<int>> gseg(kPairClasses);  // starts of the groups in order, and the end
+    for (int cl = 0; cl < kPairClasses; ++cl) {
+        const size_t o0 = order.size();
+        for (int p = 0; p < np; ++p)
+            if (c->pair_cls[p] == cl) order.push_back(p);
+        std::sort(order.begin() + o0, order.end(), [&](int x, int y) {
+            if (c->pairs[x].grp != c->pairs[y].grp) return c->pairs[x].grp > c->pairs[y].grp;
+            return c->pair_q[x] > c->pair_q[y];
+        });
+        for (size_t i = o0; i < order.size(); ++i)
+            if (i == o0 || c->pairs[order[i]].grp != c->pairs[order[i - 1]].grp) gseg[cl].push_back((int)i);
+        cbeg[cl + 1] = (int)order.size();
+        gseg[cl].push_back((int)order.size());
+    }
+    int rc;
+    if ((rc = dev_upload(&c->d_gorder, order, c->stream)) != PK_OK) return rc;
+    struct Range {
+        int start, count;
+    };
+    for (int cb = 0; cb < kPairClasses; ++cb)
+        for (int ck = 0; ck < kPairClasses; ++ck) {
+            const int nbra = cbeg[cb + 1] - cbeg[cb];
+            if (nbra == 0 || cbeg[ck + 1] == cbeg[ck]) continue;
+            std::vector<std::vector<Range>> rg(nbra);
+            parallel_for((size_t)nbra, [&](size_t t) {
+                const double qb = c->pair_q[order[cbeg[cb] + t]];
+                for (size_t g = 0; g + 1 < gseg[ck].size(); ++g) {
+                    int lo = gseg[ck][g], hi = gseg[ck][g + 1];
+                    const int g0 = lo;
+                    while (lo < hi) {
+                        const int mid = (lo + hi) / 2;
+                        if (qb * c->pair_q[order[mid]] >= c->tol)
+                            lo = mid + 1;
+                        else
+                            hi = mid;
+                    }
+                    if (lo == g0) continue;
+                    if (!rg[t].empty() && rg[t].back().start + rg[t].back().count == g0)
+                        rg[t].back().count += lo - g0;
+                    else
+                        rg[t].push_back({g0, lo - g0});
+                }
+            });
+            size_t tot = 0;
+            for (const auto &v : rg)
+                for (const Range &r : v) tot += r.count;
+            if (tot == 0) continue;
+            const pk::GradEntry &e = grad_table()[cb * kPairClasses + ck];
+            const size_t group = (std::min<size_t>(kRowKetsMax, std::max<size_t>(1, tot / kGradItems)) + e.qw - 1) / e.qw * e.qw;
+            std::vector<int> it[4];
+            std::vector<double> cost;
+            GradWork w;
+            w.cls = cb * kPairClasses + ck;
+            // steps of the item (n kets from s0): primitive quartets of the largest
+            // quartet, and the densities' share, per group of slots
+            auto steps = [&](int np, int s0, int n) {
+                return (1.0 + (double)np * c->pairs[order[s0]].nprim) * ((n + e.qw - 1) / e.qw);
+            };
+            double total = 0.0;
+            for (int t = 0; t < nbra; ++t)
+                for (const Range &r : rg[t]) total += steps(c->pairs[order[cbeg[cb] + t]].nprim, r.start, r.count);
+            const double most = std::max(32.0, total / kGradItems);  // steps of one item, about
+            for (int t = 0; t < nbra; ++t)
+                for (const Range &r : rg[t])
+                    for (int s0 = 0; s0 < r.count; s0 += (int)group) {
+                        const int n = std::min<int>((int)group, r.count - s0), b = order[cbeg[cb] + t];
+                        const int np = c->pairs[b].nprim;
+                        const double st = steps(np, r.start + s0, n);
+                        const int cuts = std::max(1, std::min(np, (int)std::ceil(st / (2.0 * most))));
+                        for (int k = 0; k < cuts; ++k) {
+                            const int p0 = (int)((int64_t)np * k / cuts), p1 = (int)((int64_t)np * (k + 1) / cuts);
+                            it[0].push_back(b);
+                            it[1].push_back(r.start + s0);
+                            it[2].push_back(n);
+                            it[3].push_back(p0 | (p1 << 16));
+                            cost.push_back(steps(p1 - p0, r.start + s0, n));
+                        }
+                    }
+            const int ni = (int)cost.size();
+            std::vector<int> o(ni), items(4 * (size_t)ni);
+            std::iota(o.begin(), o.end(), 0);
+            std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+            for (int k = 0; k < 4; ++k)
+                for (int i = 0; i < ni; ++i) items[(size_t)k * ni + i] = it[k][o[i]];
+            // queue balance: longest lists first
+            const int la = class_la(cb), lb = class_lb(cb), lc = class_la(ck), ld = class_lb(ck);
+            const double per = 20.0 + 12.0 * (la + lb + lc + ld + 1) + 6.0 * pk::nlev(lc, lc + ld);
+            for (double x : cost) w.cost += x * per * ((la + lb + lc + ld + 1) / 2 + 1);
+            w.nitems = ni;
+            if ((rc = dev_upload(&w.d_items, items, c->stream)) != PK_OK) return rc;
+            PK_HIP(hipStreamSynchronize(c->stream));  // items leaves its scope
+            c->gwork.push_back(w);
+        }
+    std::sort(c->gwork.begin(), c->gwork.end(), [](const GradWork &x, const GradWork &y) { return x.cost > y.cost; });
+    PK_HIP(hipStreamSynchronize(c->stream));
+    c->gwork_tol = c->tol;
     return PK_OK;
 }
 
@@ -1408,6 +1559,7 @@ int pk_ctx_destroy(pk_ctx *c) {
     if (!c) return PK_OK;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     free_work(c);
+    free_grad(c);
     for (void *p : {(void *)c->d_pairs, (void *)c->d_prims, (void *)c->d_Q, (void *)c->d_fnorm, (void *)c->d_P,
                     (void *)c->d_Pn, (void *)c->d_A, (void *)c->d_B, (void *)c->d_J, (void *)c->d_K, (void *)c->d_G, (void *)c->d_J2,
                     (void *)c->d_palpha, (void *)c->d_hz, (void *)c->d_B2, (void *)c->d_P32, (void *)c->d_Pk1n, (void *)c->d_Pk2n, (void *)c->d_gsh, (void *)c->d_pair_sh,
@@ -1572,7 +1724,7 @@ int pk_fock_jk_uhf(pk_ctx *c, const double *Pa, const double *Pb, double *Jt, do
 }
 
 // Two-electron gradient: the densities are scaled into the internal order,
-// then every class list of the energy build (same screening) runs through the
+// then every ordered class (same screening as the energy build) runs through its
 // derivative kernel; the per-shell sums leave through the context's buffer.
 int pk_eri_gradient(pk_ctx *c, const double *Pj, const double *Pk1, const double *Pk2, double kx, double *grad,
                     int memkind) {
@@ -1586,9 +1738,7 @@ int pk_eri_gradient(pk_ctx *c, const double *Pj, const double *Pk1, const double
     if (!c->d_Pk1n) PK_HIP(hipMalloc((void **)&c->d_Pk1n, n2));
     if (!c->d_Pk2n) PK_HIP(hipMalloc((void **)&c->d_Pk2n, n2));
     if (!c->d_gsh) PK_HIP(hipMalloc((void **)&c->d_gsh, 3 * (size_t)c->ns * sizeof(double)));
-    static const hipError_t attr = hipFuncSetAttribute(
-        (const void *)pk::k_grad, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pk::grad_lds_bytes(kMaxL, kMaxL, kMaxL, kMaxL));
-    PK_HIP(attr);
+    if ((rc = build_grad(c)) != PK_OK) return rc;
     hipStream_t s = c->stream;
     const double *src[3] = {Pj, Pk1, Pk2};
     if (memkind == PK_MEM_HOST) {
@@ -1607,14 +1757,28 @@ int pk_eri_gradient(pk_ctx *c, const double *Pj, const double *Pk1, const double
         if (src[i]) hipLaunchKernelGGL(k_scale_density, g2, dim3(256), 0, s, src[i], c->d_fnorm, dst[i], t);
     hipLaunchKernelGGL(k_fill, dim3((unsigned)((3 * c->ns + 255) / 256)), dim3(256), 0, s, c->d_gsh,
                        (size_t)3 * c->ns, 0.0);
-    for (const ClassWork &w : c->work) {
-        const ClassFns &f = kClasses[w.cls];
-        const int *wv = w.d_wave;
+    // the class lists are independent: longest first to the least loaded of the
+    // context stream and the side queues
+    hipStream_t q[kSideQueues + 1] = {s};
+    int nq = 1;
+    if (!c->side_off && c->gwork.size() > 1) {
+        if ((rc = ensure_side(c)) != PK_OK) return rc;
+        PK_HIP(hipEventRecord(c->fork_ev, s));
+        for (int i = 0; i < kSideQueues; ++i) {
+            q[nq++] = c->side[i];
+            PK_HIP(hipStreamWaitEvent(c->side[i], c->fork_ev, 0));
+        }
+    }
+    double load[kSideQueues + 1] = {};
+    const int nk = Pk2 ? 2 : 1;
+    for (const GradWork &w : c->gwork) {
+        const pk::GradEntry &e = grad_table()[w.cls];
         pk::GradArgs a{};
-        a.wave_bra = wv;
-        a.wave_start = wv + w.nwaves;
-        a.wave_count = wv + 2 * w.nwaves;
-        a.kets = w.d_kets;
+        a.item_bra = w.d_items;
+        a.item_start = w.d_items + w.nitems;
+        a.item_count = w.d_items + 2 * (size_t)w.nitems;
+        a.item_prim = w.d_items + 3 * (size_t)w.nitems;
+        a.order = c->d_gorder;
         a.pairs = c->d_pairs;
         a.prims = c->d_prims;
         a.palpha = c->d_palpha;
@@ -1622,18 +1786,30 @@ int pk_eri_gradient(pk_ctx *c, const double *Pj, const double *Pk1, const double
         a.pair_sh = c->d_pair_sh;
         a.Pj = c->d_Pn;
         a.Pk1 = c->d_Pk1n;
-        a.Pk2 = Pk2 ? c->d_Pk2n : nullptr;
+        a.Pk2 = c->d_Pk2n;
         a.Q = c->d_Q;
         a.g = c->d_gsh;
         a.tol = c->tol;
         a.kx = kx;
         a.nb = c->nb;
-        a.nitems = w.nwaves;
-        a.la = f.la;
-        a.lb = f.lb;
-        a.lc = f.lc;
-        a.ld = f.ld;
-        hipLaunchKernelGGL(pk::k_grad, dim3(w.nwaves), dim3(64), pk::grad_lds_bytes(f.la, f.lb, f.lc, f.ld), s, a);
+        a.nitems = w.nitems;
+        const void *k = nk == 2 ? e.k2 : e.k1;
+        static std::atomic<int> attr_done[2 * kPairClasses * kPairClasses];  // zero-initialised
+        std::atomic<int> &done = attr_done[2 * w.cls + nk - 1];
+        if (!done.load()) {
+            PK_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax));
+            done.store(1);
+        }
+        int j = 0;
+        for (int i = 1; i < nq; ++i)
+            if (load[i] < load[j]) j = i;
+        load[j] += w.cost;
+        void *args[] = {&a};
+        PK_HIP(hipLaunchKernel(k, dim3(w.nitems, e.rc), dim3(64), args, e.lds[nk - 1], q[j]));
+    }
+    for (int i = 1; i < nq; ++i) {
+        PK_HIP(hipEventRecord(c->join_ev[i - 1], q[i]));
+        PK_HIP(hipStreamWaitEvent(s, c->join_ev[i - 1], 0));
     }
     PK_HIP(hipGetLastError());
     const size_t gb = 3 * (size_t)c->ns * sizeof(double);

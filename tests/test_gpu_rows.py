@@ -36,3 +36,21 @@ def test_row_kernels_match_oracle(mol, basis, rows, monkeypatch):
     d = [np.abs(x).max() for x in (J - Ja, K - Ka, Jt - Ja - Jb, K1 - Ka, K2 - Kb)]
     print("%s/%s exchange rows %s: max|dJ| %.1e |dK| %.1e, UHF %.1e %.1e %.1e" % ((mol, basis, rows) + tuple(d)))
     assert max(d) < TOL
+
+
+@pytest.mark.parametrize("mol,basis", [("water", "sto-3g"), ("water2", "cc-pvdz"), ("ethane", "3-21g")])
+def test_gradient_items_match_oracle(mol, basis):
+    """Work items of the gradient: contractions cut along the bra's primitives
+    (nine s primitives in cc-pVDZ), slots left over, one and two exchange
+    densities.  Bar: 1e-9 Eh/Bohr, as for the other gradients."""
+    Z, X = MOLS[mol]()
+    Xb = np.asarray(X) * ANGSTROM_TO_BOHR
+    ref = Ref(basis, np.asarray(Z), Xb, engine="os", tol_eri=1e-11)
+    eng = FockEngine(Shells(*ref.shells()), "os", 1e-11)
+    rng = np.random.default_rng(22)
+    A, B = rng.normal(size=(2, eng.nbasis, eng.nbasis)) * 0.1
+    Pa, Pb = A + A.T, B + B.T
+    for args in ((Pa, Pa, None, 1.0), (Pa + Pb, Pa, Pb, 2.0)):
+        d = np.abs(eng.eri_gradient_atoms(Xb, *args) - ref.eri_gradient(*args)).max()
+        print("%s/%s: max|dg| %.1e" % (mol, basis, d))
+        assert d < TOL
