@@ -317,7 +317,7 @@ __global__ __launch_bounds__(64) void k_generic(GenArgs a) {
         double deg = 1.0;
         if (pb.diag) deg *= 0.5;
         if (pk.diag) deg *= 0.5;
-        if (bra == ket) deg *= 0.5;
+        if (pb.f0 == pk.f0 && pb.f1 == pk.f1) deg *= 0.5;
         const bool all_pass = pb.qmin * pk.qmin >= a.tol;
         // density (and Schwarz) blocks of the quartet into LDS: independent
         // loads issued together, read many times by the reductions below

@@ -150,6 +150,10 @@ constexpr bool seg_alt_class(int la, int lb, int lc, int ld) {
 
 // J/K kernel: one wave = one bra pair and up to 64 ket pairs.  The integrals
 // are computed in R; the J and K accumulators are FP64.
+// A pair of a work list may be a record with a part of the pair's primitives (J
+// and K are linear in them; pairs are the same when their functions are): the
+// lists cut contractions that would be one serial chain outlasting the rest of
+// the list, or that leave lanes idle.
 // NK = 2: one-pass UHF digestion, J of P (= Pa + Pb) into A and the exchange of
 // PK (= Pa) into B and of PK2 (= Pb) into B2 from the same integrals.
 //
@@ -257,7 +261,7 @@ __global__ __launch_bounds__(256) void k_jk(JKArgs a) {
         D deg = D(1);
         if (pb.diag) deg *= D(0.5);
         if (pk.diag) deg *= D(0.5);
-        if (bra == ket) deg *= D(0.5);
+        if (pb.f0 == pk.f0 && pb.f1 == pk.f1) deg *= D(0.5);
         if (!active) deg = D(0);
         // every function quartet passes the Schwarz test when the smallest
         // function-pair bounds do; otherwise each one is tested

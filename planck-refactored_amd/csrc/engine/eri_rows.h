@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256, (RowCls<LA, LB, LC, LD>::NF > 36 ? 1 : 2)) voi
     // the coefficients of its roots before the digestion of the previous group
     auto slot_ket = [&](int g, int s) { return a.kets[min(g + s, kend - 1)]; };
     int ida = 0, idb[RPL];                      // kets of the next group (phase A slot, rows)
-    int n_qoff, n_nq, n_c0[RPL], n_d0[RPL], n_diag[RPL], n_id[RPL];
+    int n_qoff, n_nq, n_c0[RPL], n_d0[RPL], n_diag[RPL];
     double n_qmin[RPL], n_cd[RPL][3];
     auto load_fields = [&](int g) {             // from ida, idb of group g
         const PairDev *pk = a.pairs + ida;
@@ -260,7 +260,6 @@ __global__ __launch_bounds__(256, (RowCls<LA, LB, LC, LD>::NF > 36 ? 1 : 2)) voi
         sfor<0, RPL>([&](auto k_) {
             constexpr int k = PK_CI(k_);
             const PairDev *pr = a.pairs + idb[k];
-            n_id[k] = idb[k];
             n_c0[k] = pr->f0;
             n_d0[k] = pr->f1;
             n_diag[k] = pr->diag;
@@ -384,7 +383,7 @@ __global__ __launch_bounds__(256, (RowCls<LA, LB, LC, LD>::NF > 36 ? 1 : 2)) voi
             kqmin[k] = n_qmin[k];
             sfor<0, 3>([&](auto q_) { cd[k][PK_CI(q_)] = n_cd[k][PK_CI(q_)]; });
             double d = n_diag[k] ? 0.5 * bdeg : bdeg;
-            if (bra == n_id[k]) d *= 0.5;
+            if (cf0[k] == bf0 && df0[k] == bf1) d *= 0.5;
             deg[k] = live[k] && g0 + sb[k] < kend ? d : 0.0;  // 0 for lanes and slots without a quartet
         });
         // densities of the group's quartets, one element of [slot][PE] per lane and load

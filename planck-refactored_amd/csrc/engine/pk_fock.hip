@@ -23,6 +23,7 @@
 #include <numeric>
 #include <string>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "eri_classes.h"
@@ -76,6 +77,15 @@ constexpr int kSegWaves = 16;
 constexpr size_t kRowItems = 4096, kRowKetsMax = 1024;
 constexpr size_t kGradItems = 8192;  // gradient work items (one wave each) of a class, about
 constexpr size_t kLdsMax = 160 * 1024;  // LDS of a CU, and of one workgroup
+// Waves are cut along the bra's primitives above 1/kCutWaves of their list's
+// steps (items of the row kernels: four times the average), and kCutSteps
+// primitive quartets (see build_work).
+constexpr double kCutWaves = 8192.0, kCutSteps = 32.0;
+constexpr int kMinSegs = 256;  // segments below which a list runs in plain mode
+// A list with fewer quartets than lanes of two waves per SIMD (quartet slots of
+// one, for the row kernels) and at least kSplitPrims primitive quartets each has
+// its kets cut along their primitives too, in at most kSplitMost parts.
+constexpr size_t kSplitLanes = 2 * 64 * 4 * 256, kSplitSlots = 4 * 256, kSplitMost = 16, kSplitPrims = 8;
 // primitive quartets per shell quartet below which a list of a pk::seg_alt_class
 // runs in segment mode (6-31G* water clusters: 11-13; cc-pVTZ alkanes: 40-80)
 constexpr double kSegAltPrim = 24.0;
@@ -327,6 +337,7 @@ struct pk_ctx {
     std::vector<int> pair_sh;    // first and second shell of each pair
     std::vector<double> Q;  // packed nb x nb blocks, normalised functions, internal order
     pk::PairDev *d_pairs = nullptr;
+    pk::PairDev *d_wpairs = nullptr;  // pairs of the work lists: the pairs, then parts of them (build_work)
     pk::PrimDev *d_prims = nullptr;
     double *d_Q = nullptr, *d_fnorm = nullptr, *d_P = nullptr, *d_Pn = nullptr, *d_A = nullptr, *d_B = nullptr;
     double *d_J = nullptr, *d_K = nullptr;
@@ -404,6 +415,8 @@ void free_work(pk_ctx *c) {
         if (w.e1) (void)hipEventDestroy(w.e1);
     }
     c->work.clear();
+    if (c->d_wpairs) (void)hipFree(c->d_wpairs);
+    c->d_wpairs = nullptr;
     c->work_ok = false;
     c->cost_learned = false;
     drop_graph(c);
@@ -492,11 +505,12 @@ int build_schwarz(pk_ctx *c) {
     return PK_OK;
 }
 
-// Runs f(i) for i in [0, n) on up to 16 host threads (dynamic chunks of 64).
+// Runs f(i) for i in [0, n) on up to 16 host threads (dynamic chunks of 64), one
+// thread per `grain` of them (starting a thread costs tens of microseconds).
 template <typename F>
-void parallel_for(size_t n, F f) {
+void parallel_for(size_t n, F f, size_t grain = 64) {
     const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    const unsigned nt = (unsigned)std::min<size_t>(hw, (n + 63) / 64);
+    const unsigned nt = (unsigned)std::min<size_t>(hw, (n + grain - 1) / grain);
     if (nt <= 1) {
         for (size_t i = 0; i < n; ++i) f(i);
         return;
@@ -551,6 +565,20 @@ int build_work(pk_ctx *c) {
             std::sort(o.begin(), o.end(), [&](int x, int y) { return okey[v[x]] < okey[v[y]]; });
         }
     });
+    // records of parts of pairs (primitives [p0, p1)), indexed after the pairs
+    std::vector<pk::PairDev> vpairs;
+    std::unordered_map<uint64_t, int> vindex;
+    auto part_of = [&](int p, int p0, int p1) {
+        if (p1 - p0 >= c->pairs[p].nprim) return p;
+        const uint64_t key = ((uint64_t)p << 24) | ((uint64_t)p0 << 12) | (uint64_t)p1;  // nprim < 2048
+        const auto it = vindex.find(key);
+        if (it != vindex.end()) return it->second;
+        pk::PairDev v = c->pairs[p];
+        v.prim_off += p0;
+        v.nprim = p1 - p0;
+        vpairs.push_back(v);
+        return vindex[key] = np + (int)vpairs.size() - 1;
+    };
     struct BraRange {
         size_t k0 = 0, k1 = 0;  // positions [k0, k1) of the q-ordered kets
         int64_t nprimq = 0;
@@ -596,7 +624,7 @@ int build_work(pk_ctx *c) {
                     BraRange &o = outs[t];
                     o.k0 = prec == PK_PREC_FP64 ? 0 : n_hi;
                     o.k1 = std::max(o.k0, prec == PK_PREC_FP64 ? n_hi : n_tol);
-                });
+                }, 1024);
                 if (rows) {
                     // about kRowItems work items of equal ket counts, whole groups
                     size_t tot = 0;
@@ -611,18 +639,12 @@ int build_work(pk_ctx *c) {
                 w.block = c->block_forced ? c->block0 : 0;
                 // offsets of every bra's kets and waves (prefix sums), then the
                 // flat arrays filled in parallel
-                std::vector<size_t> koff(tasks.size() + 1, 0), woff(tasks.size() + 1, 0);
-                for (size_t t = 0; t < tasks.size(); ++t) {
-                    const size_t n = outs[t].k1 - outs[t].k0;
-                    koff[t + 1] = koff[t] + n;
-                    woff[t + 1] = woff[t] + (n + group - 1) / group;
-                }
+                std::vector<size_t> koff(tasks.size() + 1, 0);
+                for (size_t t = 0; t < tasks.size(); ++t) koff[t + 1] = koff[t] + (outs[t].k1 - outs[t].k0);
                 if (koff.back() > (size_t)INT32_MAX) return fail(PK_ERR_ARG, "build_work: more than 2^31 quartets in one class");
-                const size_t nw = woff.back();
                 // the ket array is written entirely below: no value-initialisation
                 // (it holds one index per quartet, up to GBs for large batches)
                 std::unique_ptr<int[]> kets(new int[std::max<size_t>(1, koff.back())]);
-                std::vector<int> packed(4 * nw);
                 // pass 2: every bra's kets in ket order (ordering group
                 // descending, then first and second function) straight into the
                 // flat array, and its waves
@@ -653,13 +675,6 @@ int build_work(pk_ctx *c) {
                         o.nprimq += (int64_t)K;
                         o.flops += pk::model_flops(f.la, f.lb, f.lc, f.ld, K);
                     }
-                    size_t wi = woff[t];
-                    for (size_t s0 = 0; s0 < n; s0 += group, ++wi) {
-                        packed[wi] = b;
-                        packed[nw + wi] = (int)(koff[t] + s0);
-                        packed[2 * nw + wi] = (int)std::min<size_t>(group, n - s0);
-                        packed[3 * nw + wi] = m;
-                    }
                 });
                 for (size_t t = 0; t < tasks.size(); ++t) {
                     w.nquart += (int64_t)(outs[t].k1 - outs[t].k0);
@@ -667,15 +682,86 @@ int build_work(pk_ctx *c) {
                     w.flops += outs[t].flops;
                 }
                 if (w.nquart == 0) continue;
+                // Waves of up to `group` kets, cut along the bra's primitives where a
+                // wave would take more than about 1/kCutWaves of the list's steps.  Steps
+                // of a wave: the primitive quartets of its first ket (the longest within
+                // the ordering ratio), per group of slots.
+                const size_t per = rows ? (size_t)rows_table()[cls].qw : 64;
+                const size_t parts =
+                    w.nprimq < (int64_t)kSplitPrims * w.nquart
+                        ? 1
+                        : std::min<size_t>(kSplitMost, (rows ? kSplitSlots * per : kSplitLanes) / (size_t)w.nquart);
+                if (parts > 1) {
+                    // few quartets for the chip: every ket as its parts, neighbours
+                    std::vector<int> ex;
+                    std::vector<size_t> off(1, 0);
+                    for (size_t t = 0; t < tasks.size(); ++t) {
+                        for (size_t k = koff[t]; k < koff[t + 1]; ++k) {
+                            const int nk = c->pairs[kets[k]].nprim, m = std::max(1, std::min((int)parts, nk));
+                            for (int i = 0; i < m; ++i) ex.push_back(part_of(kets[k], nk * i / m, nk * (i + 1) / m));
+                        }
+                        off.push_back(ex.size());
+                    }
+                    if (ex.size() > (size_t)INT32_MAX) return fail(PK_ERR_ARG, "build_work: more than 2^31 quartets in one class");
+                    kets.reset(new int[ex.size()]);
+                    std::copy(ex.begin(), ex.end(), kets.get());
+                    koff.swap(off);
+                }
+                auto nprim = [&](int p) { return p < np ? c->pairs[p].nprim : vpairs[p - np].nprim; };
+                std::vector<size_t> uoff(tasks.size() + 1, 0), woff(tasks.size() + 1, 0);  // waves before and after
+                for (size_t t = 0; t < tasks.size(); ++t) uoff[t + 1] = uoff[t] + (koff[t + 1] - koff[t] + group - 1) / group;
+                const size_t grain = uoff.back() > 65536 ? 64 : 4096;
+                std::vector<double> steps(uoff.back()), tsteps(tasks.size(), 0.0);
+                auto bra_of = [&](size_t t) { return by_cls[tasks[t].first][cb][tasks[t].second]; };
+                parallel_for(tasks.size(), [&](size_t t) {
+                    const int kb = c->pairs[bra_of(t)].nprim;
+                    for (size_t u = uoff[t]; u < uoff[t + 1]; ++u) {
+                        const size_t k0 = koff[t] + (u - uoff[t]) * group, m = std::min(group, koff[t + 1] - k0);
+                        steps[u] = (double)kb * nprim(kets[k0]) * ((m + per - 1) / per);
+                        tsteps[t] += steps[u];
+                    }
+                }, grain);
+                const double most = std::max(kCutSteps, std::accumulate(tsteps.begin(), tsteps.end(), 0.0) /
+                                                            (rows ? kRowItems / 4 : kCutWaves));
+                auto cuts = [&](int kb, size_t u) { return std::max(1, std::min(kb, (int)(steps[u] / most))); };
+                parallel_for(tasks.size(), [&](size_t t) {
+                    const int kb = c->pairs[bra_of(t)].nprim;
+                    size_t n = 0;
+                    for (size_t u = uoff[t]; u < uoff[t + 1]; ++u) n += cuts(kb, u);
+                    woff[t + 1] = n;
+                }, grain);
+                for (size_t t = 0; t < tasks.size(); ++t) woff[t + 1] += woff[t];
+                const size_t nw = woff.back();
+                std::vector<int> packed(4 * nw);
+                auto fill = [&](size_t t) {
+                    const int b = bra_of(t), kb = c->pairs[b].nprim;
+                    size_t wi = woff[t];
+                    for (size_t u = uoff[t]; u < uoff[t + 1]; ++u) {
+                        const size_t k0 = koff[t] + (u - uoff[t]) * group;
+                        const int nc = cuts(kb, u);
+                        for (int k = 0; k < nc; ++k, ++wi) {
+                            packed[wi] = nc == 1 ? b : part_of(b, kb * k / nc, kb * (k + 1) / nc);
+                            packed[nw + wi] = (int)k0;
+                            packed[2 * nw + wi] = (int)std::min(group, koff[t + 1] - k0);
+                            packed[3 * nw + wi] = tasks[t].first;
+                        }
+                    }
+                };
+                auto whole = [&](size_t t) { return woff[t + 1] - woff[t] == uoff[t + 1] - uoff[t]; };
+                parallel_for(tasks.size(), [&](size_t t) {
+                    if (whole(t)) fill(t);
+                }, grain);
+                for (size_t t = 0; t < tasks.size(); ++t)
+                    if (!whole(t)) fill(t);  // part_of adds records
                 w.nwaves = (int)nw;
                 if (rows) {
                     // most expensive work items first, so that none of them ends the list
                     // alone (n-C10H22 / cc-pVTZ: (dd|dp) 5.2 -> 3.4 ms, (fd|dp) 3.1 -> 2.1 ms)
                     std::vector<double> cost(nw, 0.0);
-                    for (size_t i = 0; i < nw; ++i) {
-                        const int kb = c->pairs[packed[i]].nprim;
-                        for (int j = 0; j < packed[2 * nw + i]; ++j) cost[i] += 1.0 + kb * c->pairs[kets[packed[nw + i] + j]].nprim;
-                    }
+                    parallel_for(nw, [&](size_t i) {
+                        const int kb = nprim(packed[i]);
+                        for (int j = 0; j < packed[2 * nw + i]; ++j) cost[i] += 1.0 + kb * nprim(kets[packed[nw + i] + j]);
+                    }, 1024);
                     std::vector<int> o(nw);
                     std::iota(o.begin(), o.end(), 0);
                     std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return cost[x] > cost[y]; });
@@ -717,6 +803,12 @@ int build_work(pk_ctx *c) {
                 c->work.push_back(w);
             }
         }
+    // the lists' pairs: the context's, then the parts
+    vpairs.insert(vpairs.begin(), c->pairs.begin(), c->pairs.end());
+    {
+        int rc;
+        if ((rc = dev_upload(&c->d_wpairs, vpairs, c->stream)) != PK_OK) return rc;
+    }
     // largest classes first
     std::sort(c->work.begin(), c->work.end(), [](const ClassWork &x, const ClassWork &y) { return x.flops > y.flops; });
     // launch shapes chosen by pk_ctx_autotune for this context, if any
@@ -950,7 +1042,7 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
         a.wave_count = wv + 2 * w.nwaves;
         a.wave_mol = wv + 3 * w.nwaves;
         a.kets = w.d_kets;
-        a.pairs = c->d_pairs;
+        a.pairs = c->d_wpairs;
         a.prims = c->d_prims;
         a.hz = c->d_hz;
         a.mol_off = c->d_mol_off;
@@ -1022,6 +1114,7 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
                                 (size_t)pk::ncart(f.la) * pk::ncart(f.lb);
             a.segmode = c->seg_on && (f.seg || seg_alt) && w.nseg > 0 && rows * sizeof(double) <= kSegLdsMax;
         }
+        if (w.nseg < kMinSegs) a.segmode = 0;  // the waves of a segment run one after another
         const bool alt = seg_alt && a.segmode;  // the segment-mode variant of a plain OS class
         // lanes per workgroup: the autotuned (or PK_BLOCK) shape, else one wave
         // per workgroup for the segment-mode lists of a batch of molecules whose
@@ -1365,6 +1458,35 @@ int add_molecule(pk_ctx *c, const pk_basis_desc *d, int m) {
                     pps.push_back(pp);
                     pal.push_back(al);
                 }
+            // A shell pair on one centre: alpha_i + beta_j repeats with the roles of
+            // the two exponents swapped (s and p contractions over one set of
+            // exponents, and every shell with itself), and so do P and P - A = 0, so
+            // such primitive pairs are one with the sum of their coefficients (the
+            // gradient is linear in the exponent on A: its weighted mean).  Coefficients
+            // that nearly cancel stay apart, the mean would lose digits.
+            if (R2 == 0.0) {
+                size_t n = 0;
+                for (size_t i = 0; i < pps.size(); ++i) {
+                    size_t j = 0;
+                    for (; j < n; ++j) {
+                        const double sum = pps[j].kc + pps[i].kc;
+                        if (pps[j].zeta == pps[i].zeta && pps[j].p[0] == pps[i].p[0] && pps[j].p[1] == pps[i].p[1] &&
+                            pps[j].p[2] == pps[i].p[2] &&
+                            std::fabs(sum) >= 0.5 * std::max(std::fabs(pps[j].kc), std::fabs(pps[i].kc))) {
+                            pal[j] = (pps[j].kc * pal[j] + pps[i].kc * pal[i]) / sum;
+                            pps[j].kc = sum;
+                            break;
+                        }
+                    }
+                    if (j == n) {
+                        pps[n] = pps[i];
+                        pal[n++] = pal[i];
+                    }
+                }
+                pps.resize(n);
+                pal.resize(n);
+                for (const pk::PrimDev &pp : pps) kmax = std::max(kmax, std::fabs(pp.kc) / std::sqrt(pp.zeta));
+            }
             pp_all.push_back(std::move(pps));
             pa_all.push_back(std::move(pal));
             c->pair_sh.push_back(sa);
