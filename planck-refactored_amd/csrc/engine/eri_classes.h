@@ -117,6 +117,13 @@ constexpr bool os_available(int la, int lb, int lc, int ld) {
     return la + lb + lc + ld <= 4 && nlev(la, la + lb) * nlev(lc, lc + ld) <= 54;
 }
 
+// classes that short lists run in a row kernel: also the per-lane Rys classes
+// with a p or d first ket shell (their chunk kernels each redo the roots, and a
+// single quartet per lane is a chain of their full length)
+constexpr bool small_rows(int la, int lb, int lc, int ld) {
+    return rows_class(la, lb, lc, ld) || (!os_available(la, lb, lc, ld) && lc >= 1);
+}
+
 // dynamic LDS of a k_jk launch: the exchange rows of segment mode
 inline size_t jk_lds_bytes(const JKArgs &a, int la, int lb, int nk) {
     return a.segmode ? ((size_t)nk * (ncart(la) + ncart(lb)) * a.kcols + ncart(la) * ncart(lb)) * sizeof(double) : 0;

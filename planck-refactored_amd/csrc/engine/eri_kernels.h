@@ -170,34 +170,13 @@ constexpr bool seg_alt_class(int la, int lb, int lc, int ld) {
 // later load of the wave waits for them); this replaces ~NA ND + NB ND of them
 // per quartet by a share of one flush per segment.  J_cd stays a global atomic
 // per ket component.
-// SEGV: 1 / 0 compiles the segment-mode / plain kernel, -1 takes seg_class.
-template <typename R, int LA, int LB, int LC, int LD, int ALG, int C0, int C1, int NK = 1, int SEGV = -1>
-__global__ __launch_bounds__(256) void k_jk(JKArgs a) {
+// Waves [w_first, w_end) in strides of w_step; krow: LDS of segment mode.
+template <typename R, int LA, int LB, int LC, int LD, int ALG, int C0, int C1, int NK, bool SEG>
+__device__ __forceinline__ void jk_run(const JKArgs &a, int w_first, int w_end, int w_step, int w_lead, double *krow) {
     using K = Cls<LA, LB, LC, LD>;
     constexpr int NA = K::NA, NB = K::NB, ND = K::ND, NAB = K::NAB, NE = K::NE, NCH = C1 - C0;
     constexpr int NROW = NA + NB;
-    extern __shared__ double krow[];
-    constexpr bool SEG = SEGV >= 0 ? SEGV != 0 : seg_class(LA, LB, LC, LD);
     const bool segmode = SEG && a.segmode != 0;
-    int w_first, w_end, w_step, w_lead;
-    if (segmode) {
-        int blk = blockIdx.x;
-        if (a.remap) {
-            const int per = gridDim.x >> 3;
-            blk = (blk & 7) * per + (blk >> 3);
-        }
-        if (blk >= a.nseg) return;  // the whole workgroup
-        w_lead = a.seg[blk];
-        w_end = a.seg[blk + 1];
-        w_step = (int)(blockDim.x >> 6);
-        w_first = w_lead + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    } else {
-        const int wave = wave_index(a.remap);
-        if (wave >= a.nwaves) return;
-        w_lead = w_first = wave;
-        w_end = wave + 1;
-        w_step = 1;
-    }
     const int mol = a.wave_mol[w_lead];
     const long long moff = a.mol_off[mol];
     const int nb = a.mol_nb[mol];
@@ -427,6 +406,33 @@ __global__ __launch_bounds__(256) void k_jk(JKArgs a) {
         for (int i = threadIdx.x; i < NAB; i += blockDim.x)
             unsafeAtomicAdd(&Am[(size_t)(pb.f0 + i / NB) * nb + pb.f1 + i % NB], 2.0 * jrow[i]);
     }
+}
+
+// SEGV: 1 / 0 compiles the segment-mode / plain kernel, -1 takes seg_class.
+template <typename R, int LA, int LB, int LC, int LD, int ALG, int C0, int C1, int NK = 1, int SEGV = -1>
+__global__ __launch_bounds__(256) void k_jk(JKArgs a) {
+    extern __shared__ double krow[];
+    constexpr bool SEG = SEGV >= 0 ? SEGV != 0 : seg_class(LA, LB, LC, LD);
+    int w_first, w_end, w_step, w_lead;
+    if (SEG && a.segmode != 0) {
+        int blk = blockIdx.x;
+        if (a.remap) {
+            const int per = gridDim.x >> 3;
+            blk = (blk & 7) * per + (blk >> 3);
+        }
+        if (blk >= a.nseg) return;  // the whole workgroup
+        w_lead = a.seg[blk];
+        w_end = a.seg[blk + 1];
+        w_step = (int)(blockDim.x >> 6);
+        w_first = w_lead + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    } else {
+        const int wave = wave_index(a.remap);
+        if (wave >= a.nwaves) return;
+        w_lead = w_first = wave;
+        w_end = wave + 1;
+        w_step = 1;
+    }
+    jk_run<R, LA, LB, LC, LD, ALG, C0, C1, NK, SEG>(a, w_first, w_end, w_step, w_lead, krow);
 }
 
 }  // namespace pk

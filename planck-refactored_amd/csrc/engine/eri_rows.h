@@ -133,21 +133,15 @@ __device__ __forceinline__ T uload(const T *p) {
     return *(const __attribute__((address_space(4))) T *)(unsigned long long)p;
 }
 
+// Work item blk, row chunk chunk_y, on all waves of the workgroup; smem: its LDS.
 template <int LA, int LB, int LC, int LD, int NK>
-__global__ __launch_bounds__(256, (RowCls<LA, LB, LC, LD>::NF > 36 ? 1 : 2)) void k_rows(JKArgs a) {
+__device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, double *smem) {
     using K = Cls<LA, LB, LC, LD>;
     using S = RowCls<LA, LB, LC, LD>;
     constexpr int NA = K::NA, NB = K::NB, NC = K::NC, ND = K::ND, NAB = K::NAB, NCD = K::NCD, NF = K::NF, NR = K::NR;
     constexpr int RPL = S::RPL, QW = S::QW, RN = S::RN, RL = S::RL, NGP = S::NGP, NROW = NA + NB, GD = S::wave_doubles(NK);
     constexpr bool RUN = S::run(NK);
     constexpr int CB = QW * NK * NROW * NC;
-    extern __shared__ double smem[];
-    int blk = blockIdx.x;
-    if (a.remap) {
-        const int per = gridDim.x >> 3;
-        blk = (blk & 7) * per + (blk >> 3);
-    }
-    if (blk >= a.nwaves) return;  // the whole workgroup
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwg = (int)(blockDim.x >> 6);
@@ -190,7 +184,7 @@ __global__ __launch_bounds__(256, (RowCls<LA, LB, LC, LD>::NF > 36 ? 1 : 2)) voi
     const double lim = ax == 1 ? pk_rys_aw[pk_rys_abase[NR] + r_a] : pk_rys_ax2[pk_rys_abase[NR] + r_a];
 
     // phase B role: rows idx = lane + 64 k of (slot, row)
-    const int row0 = S::RC > 1 ? (int)blockIdx.y * RN : 0;
+    const int row0 = S::RC > 1 ? chunk_y * RN : 0;
     int sb[RPL], ro[RPL][3], af_[RPL], bf_[RPL], ka_[RPL], kb_[RPL];
     bool live[RPL];
     double Pab[RPL], Qab[RPL], jab[RPL];
@@ -605,6 +599,18 @@ __global__ __launch_bounds__(256, (RowCls<LA, LB, LC, LD>::NF > 36 ? 1 : 2)) voi
         const double x = jrow[i];
         if (x != 0.0) unsafeAtomicAdd(&Am[(size_t)(bf0 + i / NB) * nb + bf1 + i % NB], 2.0 * x);
     }
+}
+
+template <int LA, int LB, int LC, int LD, int NK>
+__global__ __launch_bounds__(256, (RowCls<LA, LB, LC, LD>::NF > 36 ? 1 : 2)) void k_rows(JKArgs a) {
+    extern __shared__ double smem[];
+    int blk = blockIdx.x;
+    if (a.remap) {
+        const int per = gridDim.x >> 3;
+        blk = (blk & 7) * per + (blk >> 3);
+    }
+    if (blk >= a.nwaves) return;  // the whole workgroup
+    rows_run<LA, LB, LC, LD, NK>(a, blk, (int)blockIdx.y, smem);
 }
 
 }  // namespace pk

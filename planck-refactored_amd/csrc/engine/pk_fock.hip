@@ -31,6 +31,7 @@
 #include "eri_grad.h"
 #include "grad_table.h"
 #include "rows_table.h"
+#include "small_table.h"
 
 // per-class launchers, defined in pk_kernels.hip
 #define PK_DECL(a, b, c, d, shard)                                                             \
@@ -81,6 +82,14 @@ constexpr size_t kLdsMax = 160 * 1024;  // LDS of a CU, and of one workgroup
 // steps (items of the row kernels: four times the average), and kCutSteps
 // primitive quartets (see build_work).
 constexpr double kCutWaves = 8192.0, kCutSteps = 32.0;
+// quartets below which the list of a class with a per-lane Rys and a row kernel
+// takes the row kernel (fewer than the lanes of two waves per SIMD)
+constexpr size_t kRowsFew = 2 * 64 * 4 * 256;
+// A build whose lists hold at most kSmallWaves waves and work items in all is
+// short: its lists go out in one launch (k_small).  H2O / 6-31G* 0.76 -> 0.07 ms,
+// three waters 1.47 -> 0.32 ms, H2O / cc-pVTZ 4.3 -> 0.72 ms; above it the lists
+// win by themselves (n-C2H6 / cc-pVTZ, 60 thousand waves, 2.6 ms against 4.9 ms).
+constexpr int64_t kSmallWaves = 32768;
 constexpr int kMinSegs = 256;  // segments below which a list runs in plain mode
 // A list with fewer quartets than lanes of two waves per SIMD (quartet slots of
 // one, for the row kernels) and at least kSplitPrims primitive quartets each has
@@ -102,6 +111,8 @@ struct ClassFns {
     int la, lb, lc, ld;
     bool has_os;    // Obara-Saika per-lane kernel
     bool has_tmpl;  // Rys per-lane kernel (else the row kernel, pk::rows_class)
+    bool few_rows;  // short lists of the class run in a row kernel (pk::small_rows)
+    int small_set;  // k_small set that covers the class (-1: none)
     bool seg;       // the per-lane kernels run in segment mode (pk::seg_class)
     bool seg_alt;   // the OS kernel also exists in segment mode (pk::seg_alt_class)
     void (*jk_os)(const pk::JKArgs &, int, int, hipStream_t, int &);
@@ -116,6 +127,7 @@ struct ClassFns {
 
 #define PK_ENTRY(a, b, c, d, shard)                                                             \
     ClassFns{a, b, c, d, pk::os_available(a, b, c, d), pk::rys_tmpl_available(a, b, c, d),      \
+             pk::small_rows(a, b, c, d), pk::small_class(a, b, c, d) ? ((a) == 3 ? 1 : 0) : -1,     \
              pk::seg_class(a, b, c, d), pk::os_available(a, b, c, d) && pk::seg_alt_class(a, b, c, d), \
              &pk_launch_jk_os_##a##b##c##d, &pk_launch_jk_rys_##a##b##c##d,                     \
              &pk_launch_jk_os32_##a##b##c##d, &pk_launch_jk_rys32_##a##b##c##d,                 \
@@ -201,6 +213,22 @@ __global__ void k_scale_density(const double *__restrict__ P, const double *__re
     Pn[o + (size_t)pr * nb + pc] = n[pr] * n[pc] * P[o + i];
 }
 
+// The same, and the accumulators of the build cleared
+__global__ void k_prepare(const double *__restrict__ P, const double *__restrict__ nrm, double *__restrict__ Pn,
+                          double *__restrict__ A, double *__restrict__ B, MolTab t) {
+    const int m = blockIdx.y, nb = t.nb[m];
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (size_t)nb * nb) return;
+    const int r = (int)(i / nb), c = (int)(i % nb);
+    const int *ps = t.pos + t.foff[m];
+    const int pr = ps[r], pc = ps[c];
+    const double *n = nrm + t.foff[m];
+    const size_t o = (size_t)t.off[m];
+    Pn[o + (size_t)pr * nb + pc] = n[pr] * n[pc] * P[o + i];
+    A[o + i] = 0.0;
+    B[o + i] = 0.0;
+}
+
 // out (caller's order) = in (internal order)
 __global__ void k_unpermute(const double *__restrict__ in, double *__restrict__ out, MolTab t) {
     const int m = blockIdx.y, nb = t.nb[m];
@@ -271,6 +299,7 @@ struct ClassWork {
     int nseg = 0;          // segments: runs of at most kSegWaves waves of one bra
     int *d_seg = nullptr;  // [nseg + 1] first wave of each segment
     int kcols = 0;         // LDS columns of an exchange row (largest molecule)
+    bool rows = false;     // runs in the class's row kernel
     int group = 0;         // row kernels: most kets of a work item
     int kernels = 0;
     double ms_total = 0.0;
@@ -349,6 +378,10 @@ struct pk_ctx {
     int *d_pair_sh = nullptr;
     std::vector<ClassWork> work;
     bool work_ok = false;
+    pk::SmallList *d_small = nullptr;  // the lists, for k_small; null when the build is not short
+    pk::SmallTab small_tab[2];
+    int small_blocks[2] = {0, 0};
+    size_t small_lds[2] = {0, 0};
     std::vector<GradWork> gwork;  // gradient work items, built by the first gradient at a tolerance
     int *d_gorder = nullptr;
     double gwork_tol = -1.0;
@@ -385,8 +418,14 @@ int list_kind(const pk_ctx *c, const ClassWork &w) {
     const ClassFns &f = kClasses[w.cls];
     const bool fp32 = w.prec == PK_PREC_MIXED && !w.alt;
     if (use_os(c, f)) return fp32 ? 3 : 0;
-    if (f.has_tmpl && !(w.alt && w.prec == PK_PREC_FP64)) return fp32 ? 4 : 1;
+    if (!w.rows && !(w.alt && w.prec == PK_PREC_FP64)) return fp32 ? 4 : 1;
     return 2;
+}
+
+// lists that k_small takes: Obara-Saika classes and rows (in FP64)
+bool small_covers(const ClassWork &w) {
+    const ClassFns &f = kClasses[w.cls];
+    return f.small_set >= 0 && (w.rows || f.has_os) && w.prec == PK_PREC_FP64;
 }
 
 void drop_graph(pk_ctx *c) {
@@ -417,6 +456,8 @@ void free_work(pk_ctx *c) {
     c->work.clear();
     if (c->d_wpairs) (void)hipFree(c->d_wpairs);
     c->d_wpairs = nullptr;
+    if (c->d_small) (void)hipFree(c->d_small);
+    c->d_small = nullptr;
     c->work_ok = false;
     c->cost_learned = false;
     drop_graph(c);
@@ -588,11 +629,7 @@ int build_work(pk_ctx *c) {
         for (int ck = 0; ck <= cb; ++ck) {
             const int cls = quart_class(cb, ck);
             const ClassFns &f = kClasses[cls];
-            const bool rows = !f.has_tmpl;
-            const bool split = mixed && !rows;
-            // kets per work item: a wave of 64 lanes for the per-lane kernels;
-            // for the row kernels a workgroup's share of a bra's kets (below)
-            size_t group = 64;
+            const bool split = mixed && f.has_tmpl;
             // bra tasks of every molecule, in order
             std::vector<std::pair<int, int>> tasks;
             for (int m = 0; m < c->nmol; ++m)
@@ -625,6 +662,16 @@ int build_work(pk_ctx *c) {
                     o.k0 = prec == PK_PREC_FP64 ? 0 : n_hi;
                     o.k1 = std::max(o.k0, prec == PK_PREC_FP64 ? n_hi : n_tol);
                 }, 1024);
+                // kets per work item: a wave of 64 lanes for the per-lane kernels; for
+                // the row kernels a workgroup's share of a bra's kets (below)
+                size_t group = 64;
+                // row kernel: by class, or a short list of a class that has both
+                bool rows = !f.has_tmpl;
+                if (f.few_rows && !mixed) {
+                    size_t tot = 0;
+                    for (const BraRange &o : outs) tot += o.k1 - o.k0;
+                    rows = rows || tot < kRowsFew;
+                }
                 if (rows) {
                     // about kRowItems work items of equal ket counts, whole groups
                     size_t tot = 0;
@@ -636,6 +683,7 @@ int build_work(pk_ctx *c) {
                 ClassWork w;
                 w.cls = cls;
                 w.prec = prec;
+                w.rows = rows;
                 w.block = c->block_forced ? c->block0 : 0;
                 // offsets of every bra's kets and waves (prefix sums), then the
                 // flat arrays filled in parallel
@@ -819,6 +867,33 @@ int build_work(pk_ctx *c) {
                 w.remap = t.remap;
                 w.alt = t.alt;
             }
+    // a short build: its lists for k_small
+    int64_t waves = 0;
+    for (const ClassWork &w : c->work) waves += w.nwaves;
+    std::vector<pk::SmallList> small;  // uploaded from here until the synchronisation below
+    if (waves <= kSmallWaves && !mixed && c->tuned.empty() && !c->block_forced) {
+        c->small_tab[0].n = c->small_tab[1].n = 0;
+        c->small_blocks[0] = c->small_blocks[1] = 0;
+        c->small_lds[0] = c->small_lds[1] = 0;
+        for (size_t i = 0; i < c->work.size(); ++i) {
+            const ClassWork &w = c->work[i];
+            const ClassFns &f = kClasses[w.cls];
+            const pk::RowsEntry &r = rows_table()[w.cls];
+            pk::SmallList l{w.d_wave, w.d_kets, w.nwaves, w.cls, 1};
+            if (w.rows) l.chunk = std::max(1, std::min(8, (w.group + r.qw - 1) / r.qw / 2));
+            small.push_back(l);
+            if (!small_covers(w)) continue;
+            pk::SmallTab &t = c->small_tab[f.small_set];
+            t.first[t.n] = c->small_blocks[f.small_set];
+            t.list[t.n++] = (int)i;
+            c->small_blocks[f.small_set] += w.nwaves * (w.rows ? r.rc : 1);
+            if (w.rows)
+                c->small_lds[f.small_set] = std::max(
+                    c->small_lds[f.small_set], (size_t)r.wave_bytes[0] + (size_t)pk::ncart(f.la) * pk::ncart(f.lb) * sizeof(double));
+        }
+        int rc;
+        if ((rc = dev_upload(&c->d_small, small, c->stream)) != PK_OK) return rc;
+    }
     PK_HIP(hipStreamSynchronize(c->stream));
     if (c->st.quartets >= kSideMinQuartets) {
         int rc;
@@ -985,9 +1060,53 @@ int ensure_side(pk_ctx *c) {
     return PK_OK;
 }
 
+// kernel arguments of a build, without those of a list
+pk::JKArgs build_args(const pk_ctx *c, const BuildBufs &sb) {
+    pk::JKArgs a{};
+    a.pairs = c->d_wpairs;
+    a.prims = c->d_prims;
+    a.hz = c->d_hz;
+    a.mol_off = c->d_mol_off;
+    a.mol_nb = c->d_mol_nb;
+    a.P = sb.Pn;
+    a.P32 = sb.P32;
+    a.PK = sb.PKa;
+    a.PK2 = sb.PKb;
+    a.Q = c->d_Q;
+    a.A = sb.A;
+    a.B = sb.B;
+    a.B2 = sb.B2;
+    a.tol = c->tol;
+    a.tblk = c->d_tblk;
+    return a;
+}
+
+// The lists of a short build that k_small covers, in one launch (two with f
+// shells); the rest one by one.
+int launch_small(pk_ctx *c, const BuildBufs &sb, int &nl) {
+    static const void *const kernel[2] = {pk_small_kernel<0>(), pk_small_kernel<1>()};
+    static const hipError_t attr[2] = {
+        hipFuncSetAttribute(kernel[0], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax),
+        hipFuncSetAttribute(kernel[1], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax)};
+    pk::JKArgs a = build_args(c, sb);
+    const pk::SmallList *lists = c->d_small;
+    for (int k = 0; k < 2; ++k) {
+        if (c->small_tab[k].n == 0) continue;
+        PK_HIP(attr[k]);
+        void *args[] = {&a, &lists, &c->small_tab[k]};
+        PK_HIP(hipLaunchKernel(kernel[k], dim3(c->small_blocks[k]), dim3(64), args, c->small_lds[k], c->stream));
+        ++nl;
+    }
+    int rc;
+    for (ClassWork &w : c->work)
+        if (!small_covers(w) && (rc = launch_list(c, w, sb, false, c->stream, nl)) != PK_OK) return rc;
+    return PK_OK;
+}
+
 int launch_classes(pk_ctx *c, const BuildBufs &sb, bool events, int &nl) {
     int rc;
     hipStream_t s = c->stream;
+    if (!events && c->d_small && c->engine != PK_ENGINE_RYS && !sb.B2) return launch_small(c, sb, nl);
     // Concurrent queues (not while profiling: the class events time one list
     // at a time): lists in descending model cost, each to the queue with the
     // least cost so far, so that the small classes fill the tails of the
@@ -1036,30 +1155,15 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
     int rc;
     {
         const int *wv = w.d_wave;
-        pk::JKArgs a{};
+        pk::JKArgs a = build_args(c, sb);
         a.wave_bra = wv;
         a.wave_start = wv + w.nwaves;
         a.wave_count = wv + 2 * w.nwaves;
         a.wave_mol = wv + 3 * w.nwaves;
         a.kets = w.d_kets;
-        a.pairs = c->d_wpairs;
-        a.prims = c->d_prims;
-        a.hz = c->d_hz;
-        a.mol_off = c->d_mol_off;
-        a.mol_nb = c->d_mol_nb;
-        a.P = sb.Pn;
-        a.P32 = sb.P32;
-        a.PK = sb.PKa;
-        a.PK2 = sb.PKb;
-        a.Q = c->d_Q;
-        a.A = sb.A;
-        a.B = sb.B;
-        a.B2 = sb.B2;
-        a.tol = c->tol;
         a.nwaves = w.nwaves;
         a.remap = w.remap;
         a.seg = w.d_seg;
-        a.tblk = c->d_tblk;
         a.nseg = w.nseg;
         a.kcols = w.kcols;
         const bool uhf = sb.B2 != nullptr;
@@ -1076,7 +1180,7 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
         // compiled both ways take it for lists of few primitive quartets per
         // shell quartet (atomic-bound), the plain kernel otherwise
         const bool seg_alt = f.seg_alt && use_os(c, f) && (double)w.nprimq <= c->seg_alt_prim * (double)w.nquart;
-        if (!f.has_tmpl) {
+        if (w.rows) {
             const pk::RowsEntry &r = rows_table()[w.cls];
             const int rk = uhf ? 2 : 1;
             const size_t wave_bytes = r.wave_bytes[rk - 1];
@@ -1188,10 +1292,8 @@ int launch_build(pk_ctx *c, const double *dP, double *dJ, double *dK, double *dG
     const MolTab t{c->d_mol_off, c->d_mol_nb, c->d_mol_foff, c->d_fpos};
     const dim3 g2((unsigned)(((size_t)c->nbmax * c->nbmax + 255) / 256), (unsigned)c->nmol);
     const int gf = (int)((c->n2 + 255) / 256);
-    hipLaunchKernelGGL(k_scale_density, g2, dim3(256), 0, s, dP, c->d_fnorm, sb.Pn, t);
-    hipLaunchKernelGGL(k_fill, dim3(gf), dim3(256), 0, s, sb.A, c->n2, 0.0);
-    hipLaunchKernelGGL(k_fill, dim3(gf), dim3(256), 0, s, sb.B, c->n2, 0.0);
-    int nl = 3;
+    hipLaunchKernelGGL(k_prepare, g2, dim3(256), 0, s, dP, c->d_fnorm, sb.Pn, sb.A, sb.B, t);
+    int nl = 1;
     if (c->precision == PK_PREC_MIXED) {
         if (!sb.P32) return fail(PK_ERR_STATE, "mixed precision build without an FP32 density buffer");
         hipLaunchKernelGGL(k_to_f32, dim3(gf), dim3(256), 0, s, sb.Pn, sb.P32, c->n2);

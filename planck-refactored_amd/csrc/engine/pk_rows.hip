@@ -8,10 +8,11 @@ namespace {
 
 template <int A, int B, int C, int D, int CLS>
 void add(pk::RowsEntry *table) {
-    if constexpr (CLS % PK_NROWSHARDS == PK_SHARD && pk::rows_class(A, B, C, D)) {
+    if constexpr (CLS % PK_NROWSHARDS == PK_SHARD && pk::small_rows(A, B, C, D)) {
         using S = pk::RowCls<A, B, C, D>;
         table[CLS] = pk::RowsEntry{(const void *)pk::k_rows<A, B, C, D, 1>, (const void *)pk::k_rows<A, B, C, D, 2>,
-                                   {(int)(S::wave_doubles(1) * sizeof(double)), (int)(S::wave_doubles(2) * sizeof(double))}, S::QW, S::RC};
+                                   {(int)(S::wave_doubles(1) * sizeof(double)), (int)(S::wave_doubles(2) * sizeof(double))},
+                                   S::QW, S::RC};
     }
 }
 

@@ -54,3 +54,31 @@ def test_gradient_items_match_oracle(mol, basis):
         d = np.abs(eng.eri_gradient_atoms(Xb, *args) - ref.eri_gradient(*args)).max()
         print("%s/%s: max|dg| %.1e" % (mol, basis, d))
         assert d < TOL
+
+
+@pytest.mark.parametrize("mol,basis", [("water", "sto-3g"), ("water", "cc-pvtz"), ("water2", "cc-pvdz"), ("ethane", "6-31g*")])
+def test_short_build_in_one_launch_equals_its_lists(mol, basis):
+    """A short build goes out in one launch; with per-class timing on, its lists
+    run one by one in their own kernels.  Both must agree to the rounding of
+    another summation order (1e-12), with a density that changes in between and
+    on repeated calls, and replayed from a graph."""
+    Z, X = MOLS[mol]()
+    ref = Ref(basis, np.asarray(Z), np.asarray(X) * ANGSTROM_TO_BOHR, engine="os", tol_eri=1e-11)
+    eng = FockEngine(Shells(*ref.shells()), "os", 1e-11)
+    rng = np.random.default_rng(23)
+    for rep in range(3):
+        A = rng.normal(size=(eng.nbasis, eng.nbasis)) * 0.2
+        P = A + A.T
+        eng.profile(True)
+        J0, K0 = eng.jk(P)
+        eng.profile(False)
+        J1, K1 = eng.jk(P)
+        eng.set_graph(True)
+        J2, K2 = eng.jk(P)
+        eng.set_graph(False)
+        d = [np.abs(x).max() for x in (J1 - J0, K1 - K0, J2 - J0, K2 - K0)]
+        print("%s/%s: |dJ| %.1e |dK| %.1e, graph %.1e %.1e" % ((mol, basis) + tuple(d)))
+        assert max(d) < 1e-12 * max(1.0, np.abs(J0).max())
+        # prepare, s/p/d lists, f lists, finalize, and the five classes outside the
+        # launch: (fd|ss), (ff|ss), (fd|fd), (ff|fd), (ff|ff)
+        assert eng.stats()["kernel_launches"] <= 9
