@@ -19,7 +19,7 @@
 #define PK_RYS_COEF_QUALIFIER static __device__ const
 #include "rys_table.inc"
 #define PK_BOYS_QUALIFIER static __device__ const
-#include "boys_table.inc"
+#include "boys_poly.inc"
 
 // PrimDev::kc carries K_ab sqrt(zeta) (4/pi)^(1/4), so that the product of a bra
 // and a ket record times 1/sqrt(zeta+eta) is K_ab K_cd 2 sqrt(rho/pi).
@@ -71,29 +71,34 @@ __device__ __forceinline__ PrimQ<R> prim_quartet(const PrimDev &p, const PrimDev
 }
 
 // ---------------------------------------------------------------- Boys
-// F_0..F_M(T): 8-term Taylor series of F_M about the nearest grid point
-// (step 1/16) and downward recursion below 50, with e^{-T} = e^{-x_i} e^{-d};
-// F_0 = sqrt(pi/T)/2 and the upward recursion at and above 50.  The upward
-// recursion's e^{-T} term is dropped for M <= 4 (the orders of the
-// Obara-Saika kernels): there it is below 2e-17 of F_M, and the large-T
-// branch then costs a reciprocal square root and M products instead of an
-// exponential.
+// F_0..F_M(T), M <= 4 (the orders of the Obara-Saika kernels).  Below 50: F_M
+// from the degree-6 polynomial of the interval of width 1/16 (boys_poly.inc; its
+// error is below 4e-17 of F_M), the lower orders by the downward recursion with
+// e^{-T} = e^{-x_i} e^{-d}.  At and above 50: F_0 = sqrt(pi/T)/2 and the upward
+// recursion without its e^{-T} term, which is below 2e-17 of F_M there.
+// The loads of the interval's row bound the kernels of few integrals (every lane
+// has its own T): (ps|ss) had its texture-address unit busy 70 % of the time and
+// its vector unit 38 %.  One row per order and interval, one aligned half of a cache
+// line with e^{-x_i} in it, asks for four 16-byte loads of one line where a
+// Taylor row inside a table of all orders (192-byte rows of unaligned starts) and
+// a second table took six of up to three lines, and the Taylor factors 1/k six
+// products.  n-C10H22 / cc-pVTZ: (ps|ss) 7.7 -> 6.8 ms, (ps|ps) 5.8 -> 5.4 ms,
+// (ds|ss) 3.9 -> 3.7 ms; (ss|ss) 68 -> 58 registers.
 template <int M>
 __device__ __forceinline__ void boys(double T, double (&F)[M + 1]) {
-    static_assert(M + 8 <= PK_BOYS_COLS, "Boys table too narrow for this class");
+    static_assert(M < PK_BOYS_ORDERS, "no Boys polynomials of this order");
     if (T < (double)PK_BOYS_XMAX) {
         const int i = (int)fma(T, (double)PK_BOYS_STEP_INV, 0.5);
         const double d = fma((double)i, -1.0 / PK_BOYS_STEP_INV, T);
-        // 24-bit multiply (full rate; i < 2^24)
-        const double *row = pk_boys_table + __umul24((unsigned)i, PK_BOYS_COLS) + M;
-        double s = row[7];
-        s = fma(s, -d * (1.0 / 7.0), row[6]);
-        s = fma(s, -d * (1.0 / 6.0), row[5]);
-        s = fma(s, -d * (1.0 / 5.0), row[4]);
-        s = fma(s, -d * (1.0 / 4.0), row[3]);
-        s = fma(s, -d * (1.0 / 3.0), row[2]);
-        s = fma(s, -d * (1.0 / 2.0), row[1]);
-        s = fma(s, -d, row[0]);
+        const double2 *row = (const double2 *)(pk_boys_row + 8 * (size_t)M * PK_BOYS_ROWS) + 4 * i;
+        const double2 c01 = row[0], c23 = row[1], c45 = row[2], c6e = row[3];
+        double s = c6e.x;
+        s = fma(s, d, c45.y);
+        s = fma(s, d, c45.x);
+        s = fma(s, d, c23.y);
+        s = fma(s, d, c23.x);
+        s = fma(s, d, c01.y);
+        s = fma(s, d, c01.x);
         F[M] = s;
         if constexpr (M > 0) {
             // e^{-d}, |d| <= 1/32: 8 Taylor terms (next term < 1e-17)
@@ -105,7 +110,7 @@ __device__ __forceinline__ void boys(double T, double (&F)[M + 1]) {
             e = fma(e, -d, 0.5);
             e = fma(e, -d, 1.0);
             e = fma(e, -d, 1.0);
-            const double eT = pk_boys_exp[i] * e;
+            const double eT = c6e.y * e;
             const double t2 = 2.0 * T;
             sfor_down<M, 0>([&](auto m_) {
                 constexpr int m = PK_CI(m_);
@@ -117,37 +122,29 @@ __device__ __forceinline__ void boys(double T, double (&F)[M + 1]) {
         F[0] = 0.88622692545275801365 * r;  // sqrt(pi/T)/2
         if constexpr (M > 0) {
             const double it2 = 0.5 * r * r;
-            if constexpr (M <= 4) {
-                sfor<1, M + 1>([&](auto m_) {
-                    constexpr int m = PK_CI(m_);
-                    F[m] = (2 * m - 1) * F[m - 1] * it2;
-                });
-            } else {
-                const double eT = exp(-T);
-                sfor<1, M + 1>([&](auto m_) {
-                    constexpr int m = PK_CI(m_);
-                    F[m] = ((2 * m - 1) * F[m - 1] - eT) * it2;
-                });
-            }
+            sfor<1, M + 1>([&](auto m_) {
+                constexpr int m = PK_CI(m_);
+                F[m] = (2 * m - 1) * F[m - 1] * it2;
+            });
         }
     }
 }
 
-// FP32 path: 5-term series from the float tables below 50 (|d| <= 1/32, next
-// term below 3e-10 relative); the large-T branch in FP64 without the e^{-T}
-// term (below 2e-17 of F_M for M <= 4, the orders of the FP32 kernels).
+// FP32 path: degree-4 polynomials in float rows below 50 (error below 2e-11 of
+// F_M); the large-T branch in FP64.
 template <int M>
 __device__ __forceinline__ void boys(float T, float (&F)[M + 1]) {
-    static_assert(M + 5 <= PK_BOYS_COLS, "Boys table too narrow for this class");
+    static_assert(M < PK_BOYS_ORDERS, "no Boys polynomials of this order");
     if (T < (float)PK_BOYS_XMAX) {
         const int i = (int)fmaf(T, (float)PK_BOYS_STEP_INV, 0.5f);
         const float d = fmaf((float)i, -1.0f / PK_BOYS_STEP_INV, T);
-        const float *row = pk_boys_table_f + __umul24((unsigned)i, PK_BOYS_COLS) + M;
-        float s = row[4];
-        s = fmaf(s, -d * (1.0f / 4.0f), row[3]);
-        s = fmaf(s, -d * (1.0f / 3.0f), row[2]);
-        s = fmaf(s, -d * (1.0f / 2.0f), row[1]);
-        s = fmaf(s, -d, row[0]);
+        const float4 *row = (const float4 *)(pk_boys_row_f + 8 * (size_t)M * PK_BOYS_ROWS) + 2 * i;
+        const float4 c03 = row[0], c4e = row[1];
+        float s = c4e.x;
+        s = fmaf(s, d, c03.w);
+        s = fmaf(s, d, c03.z);
+        s = fmaf(s, d, c03.y);
+        s = fmaf(s, d, c03.x);
         F[M] = s;
         if constexpr (M > 0) {
             float e = fmaf(-d, 1.0f / 120.0f, 1.0f / 24.0f);
@@ -155,7 +152,7 @@ __device__ __forceinline__ void boys(float T, float (&F)[M + 1]) {
             e = fmaf(e, -d, 0.5f);
             e = fmaf(e, -d, 1.0f);
             e = fmaf(e, -d, 1.0f);
-            const float eT = pk_boys_exp_f[i] * e;
+            const float eT = c4e.w * e;
             const float t2 = 2.0f * T;
             sfor_down<M, 0>([&](auto m_) {
                 constexpr int m = PK_CI(m_);
@@ -168,7 +165,6 @@ __device__ __forceinline__ void boys(float T, float (&F)[M + 1]) {
         double f = 0.88622692545275801365 * r;
         F[0] = (float)f;
         if constexpr (M > 0) {
-            static_assert(M <= 4, "FP32 large-T Boys branch drops e^{-T}: orders up to 4 only");
             const double it2 = 0.5 * r * r;
             sfor<1, M + 1>([&](auto m_) {
                 constexpr int m = PK_CI(m_);

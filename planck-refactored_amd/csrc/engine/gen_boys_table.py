@@ -1,23 +1,15 @@
 #!/usr/bin/env python3
-"""Generate boys_table.inc: F_m(x_i) for the device Boys function.
+"""Generate boys_table.inc: F_m(x_i) on a grid, the table that the tests check
+the large-argument branch, the recursions and the grid values against.
 
 Grid x_i = i / 16, i = 0..BOYS_ROWS-1 (x <= 50), orders m = 0..BOYS_COLS-1, each
 value the double nearest to F_m(x_i) = gamma_inc(m + 1/2, x_i) / (2 x_i^(m+1/2))
-computed with 40-digit arithmetic (mpmath).  The kernels evaluate the top order
-by an 8-term Taylor series about the nearest grid point (|dx| <= 1/32, next term
-below 3e-17 relative) and the lower orders by the stable downward recursion
-F_{m-1} = (2 x F_m + e^{-x}) / (2m - 1).  For x >= 50 the kernels use
-F_0 = sqrt(pi/x)/2 and the upward recursion, without its e^{-x} term for
-orders m <= 4 (the only orders the Obara-Saika kernels use; the term is below
-2e-17 of F_m there).
-The FP32 kernels read float copies of both tables (nearest floats of the same
-values) with a 5-term series.
+computed with 40-digit arithmetic (mpmath), and e^{-x_i}.  The kernels read the
+polynomials of boys_poly.inc (gen_boys_poly.py) instead.
 """
 import os
-import struct
 
 import mpmath
-import numpy as np
 
 STEP_INV = 16
 XMAX = 50
@@ -29,15 +21,6 @@ def F(m, x):
     if x == 0:
         return mpmath.mpf(1) / (2 * m + 1)
     return mpmath.gammainc(m + mpmath.mpf(1) / 2, 0, x) / (2 * x ** (m + mpmath.mpf(1) / 2))
-
-
-def f32(v):
-    """C literal of the float nearest to v (v an mpf, rounded once)."""
-    r = float(struct.unpack("f", struct.pack("f", float(v)))[0])
-    # float(v) rounds to double first; correct a double-rounding tie if any
-    lo, hi = np.nextafter(np.float32(r), np.float32(-np.inf)), np.nextafter(np.float32(r), np.float32(np.inf))
-    best = min((np.float32(lo), np.float32(r), np.float32(hi)), key=lambda c: abs(mpmath.mpf(float(c)) - v))
-    return float(best).hex() + "f"
 
 
 def main():
@@ -69,15 +52,6 @@ def main():
     lines.append("// e^{-x_i} on the same grid")
     lines.append("PK_BOYS_QUALIFIER double pk_boys_exp[%d] = {" % ROWS)
     lines.append("  " + ", ".join(float(mpmath.exp(-mpmath.mpf(i) / STEP_INV)).hex() for i in range(ROWS)))
-    lines.append("};")
-    # single-precision copies (nearest floats) for the FP32 kernels
-    lines.append("// the same tables rounded to the nearest float")
-    lines.append("PK_BOYS_QUALIFIER float pk_boys_table_f[%d] = {" % (ROWS * COLS))
-    for i in range(ROWS):
-        lines.append("  " + ", ".join(f32(v) for v in rows[i]) + ",")
-    lines.append("};")
-    lines.append("PK_BOYS_QUALIFIER float pk_boys_exp_f[%d] = {" % ROWS)
-    lines.append("  " + ", ".join(f32(mpmath.exp(-mpmath.mpf(i) / STEP_INV)) for i in range(ROWS)))
     lines.append("};")
     with open(out, "w") as f:
         f.write("\n".join(lines) + "\n")
