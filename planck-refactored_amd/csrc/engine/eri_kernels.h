@@ -50,7 +50,7 @@ struct JKArgs {
     int remap;  // 1: each XCD takes a contiguous range of waves (grid a multiple of 8)
     // segment mode (see k_jk): segments of waves of one bra, block starts of
     // the function types per molecule, LDS columns per exchange row
-    const int *__restrict__ seg;   // [nseg + 1] first wave of each segment
+    const int *__restrict__ seg;   // [2 * nseg] first wave of each segment and its end
     const int *__restrict__ tblk;  // [5 * nmol]: first function of type s, p, d, f, and nb
     int nseg;
     int kcols;
@@ -125,25 +125,26 @@ __device__ __forceinline__ void os_values(const PairDev &pb, const PairDev &pk, 
 }
 
 // Classes whose per-lane kernel runs in segment mode (LDS exchange rows, see
-// k_jk).  Measured per class on n-C10H22 / cc-pVTZ (segment mode / plain):
-// kets with a p or d second shell 0.26-0.83 (the Rys classes (30|22) 0.26,
-// (30|21) 0.31, (21|11) 0.43); kets (ss) under a d or f bra 0.75-0.83; but
-// (00|00) 1.61, kets (ds) 1.16-1.30 except (20|20) 0.86, kets (fs) 1.05-2.02,
-// and the (ff| bras (20 exchange rows, few kets per bra) 1.10-2.02.
+// k_jk).  Measured per class on n-C10H22 / cc-pVTZ (segment mode / plain): kets
+// with a p or d second shell 0.26-0.83 (the Rys classes (30|22) 0.26, (30|21) 0.31,
+// (21|11) 0.43); kets (ps) and (ss) 0.60-0.83 ((ps|ps) 5.5 -> 3.9 ms, (pp|ss) 2.7 ->
+// 2.0 ms) with the most expensive segments first; but (00|00) 1.51, (10|00) 1.00
+// (n-C20H42 / cc-pVDZ 1.16), kets (ds) 1.16-1.30 except (20|20) 0.86, kets (fs)
+// 1.05-2.02, and the (ff| bras (20 exchange rows, few kets per bra) 1.10-2.02.
 constexpr bool seg_class(int la, int lb, int lc, int ld) {
     if (la == 3 && lb == 3) return false;
     if (ld >= 1) return true;
-    if (lc == 1) return la >= 1 && !(la == 1 && lb == 0);
-    if (lc == 0) return la >= 2;
+    if (lc == 1) return true;
+    if (lc == 0) return la >= 2 || lb == 1;
     return la == 2 && lb == 0 && lc == 2;
 }
 
 // Classes whose plain kernel is also compiled in segment mode, chosen at run
-// time for lists of few primitive quartets per shell quartet: (ss|ss), (ps|ss),
-// (ps|ps), (pp|ss).  In 6-31G* water clusters (about 11-13 primitive quartets
-// per shell quartet) they do ~5 exchange atomics per quartet and are bound by
-// atomic throughput; in cc-pVTZ alkanes (40-80) by the primitive loop, where
-// the plain kernel is faster.
+// time for lists of few primitive quartets per shell quartet: (ss|ss) and
+// (ps|ss).  In 6-31G* water clusters (about 11-13 primitive quartets per shell
+// quartet) they do ~5 exchange atomics per quartet and are bound by atomic
+// throughput; in cc-pVTZ alkanes (40-80) by the primitive loop, where the plain
+// kernel is faster.
 constexpr bool seg_alt_class(int la, int lb, int lc, int ld) {
     return !seg_class(la, lb, lc, ld) && la + lb + lc + ld <= 2;
 }
@@ -158,7 +159,7 @@ constexpr bool seg_alt_class(int la, int lb, int lc, int ld) {
 // PK (= Pa) into B and of PK2 (= Pb) into B2 from the same integrals.
 //
 // Segment mode (a.segmode): the waves of a workgroup take the waves
-// [seg[s], seg[s + 1]) of one bra pair, in strides of the waves per workgroup.
+// [seg[2 s], seg[2 s + 1]) of one bra pair, in strides of the waves per workgroup.
 // Every exchange contribution then lands in a row of the bra's two shells
 // (B_ac, B_ad: rows a; B_bc, B_bd: rows b) and in a column of the kets' two
 // shell types (internal order: a molecule's functions grouped by type,
@@ -421,8 +422,8 @@ __global__ __launch_bounds__(256) void k_jk(JKArgs a) {
             blk = (blk & 7) * per + (blk >> 3);
         }
         if (blk >= a.nseg) return;  // the whole workgroup
-        w_lead = a.seg[blk];
-        w_end = a.seg[blk + 1];
+        w_lead = a.seg[2 * blk];
+        w_end = a.seg[2 * blk + 1];
         w_step = (int)(blockDim.x >> 6);
         w_first = w_lead + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     } else {

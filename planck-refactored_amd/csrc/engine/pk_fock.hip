@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cmath>
 #include <cstdio>
@@ -69,9 +70,14 @@ constexpr double kPrimCut = 1e-17;  // primitive-pair screening bound (see add_m
 // (GPU_MAX_HW_QUEUES is 4: one queue per stream).
 constexpr int kSideQueues = 3;
 constexpr int64_t kSideMinQuartets = 1 << 20;
-// Segment mode of the per-lane kernels (see k_jk): at most kSegWaves waves of
-// one bra per segment, and at most kSegLdsMax bytes of LDS exchange rows.
-constexpr int kSegWaves = 16;
+// Segment mode of the per-lane kernels (see k_jk): at most kSegWaves waves of one
+// bra per segment, fewer (kSegWavesMin at least) where a list would have less than
+// kSegs of them or one would take more than 1/kSegs of the list's primitive steps,
+// and at most kSegLdsMax bytes of LDS exchange rows.  The waves of a segment run
+// one after another on its workgroup: with workgroups of two waves on n-C10H22 /
+// cc-pVTZ, 16 -> 4 waves: (pp|ss) 2.7 -> 1.6 ms, (fs|ss) 1.5 -> 1.0, but (dp|ps)
+// 6.5 -> 7.0 (every segment flushes its rows).
+constexpr size_t kSegWaves = 16, kSegWavesMin = 4, kSegs = 4096;
 // Row kernels: a list is cut into about kRowItems work items (workgroups) of at
 // most kRowKetsMax kets; measured on n-C10H22 / cc-pVTZ, 8192 items: the same or
 // up to 1.6x slower (a workgroup flushes its exchange rows once).
@@ -101,8 +107,12 @@ constexpr double kSegAltPrim = 24.0;
 constexpr size_t kSegLdsMax = 64 * 1024;
 // lanes per workgroup of a class list until pk_ctx_autotune picks its own;
 // one wave per workgroup for the segment-mode lists of a batch with at most
-// kSegOneWaveLds bytes of exchange rows (see launch_list)
-constexpr int kDefaultBlock = 256;
+// kSegOneWaveLds bytes of exchange rows (see launch_list).  128 against 256 lanes: the
+// lists one after another take the same time (n-C10H22 / cc-pVTZ 131 ms both), a
+// build over the side queues, where workgroups of several lists share a CU,
+// 117 ms against 121 (n-C20H42 / cc-pVDZ 31.5 ms against 33.9).
+constexpr int kDefaultBlock = 128;
+constexpr int kRowWavesMax = 4;  // waves per workgroup of the row kernels
 constexpr size_t kSegOneWaveLds = 24 * 1024;
 constexpr int kPairClasses = (kMaxL + 1) * (kMaxL + 2) / 2;
 constexpr int kQuartClasses = kPairClasses * (kPairClasses + 1) / 2;
@@ -296,8 +306,9 @@ struct ClassWork {
     double flops = 0.0;
     int *d_wave = nullptr;  // [4][nwaves]: bra, start, count, molecule
     int *d_kets = nullptr;
+    int row_waves[2] = {0, 0};  // row kernels: waves per workgroup, one and two exchange densities (0: not chosen yet)
     int nseg = 0;          // segments: runs of at most kSegWaves waves of one bra
-    int *d_seg = nullptr;  // [nseg + 1] first wave of each segment
+    int *d_seg = nullptr;  // [2 nseg] first wave and end of each segment, most expensive first
     int kcols = 0;         // LDS columns of an exchange row (largest molecule)
     bool rows = false;     // runs in the class's row kernel
     int group = 0;         // row kernels: most kets of a work item
@@ -781,6 +792,7 @@ int build_work(pk_ctx *c) {
                 for (size_t t = 0; t < tasks.size(); ++t) woff[t + 1] += woff[t];
                 const size_t nw = woff.back();
                 std::vector<int> packed(4 * nw);
+                std::vector<float> wsteps(nw);  // steps of every wave
                 auto fill = [&](size_t t) {
                     const int b = bra_of(t), kb = c->pairs[b].nprim;
                     size_t wi = woff[t];
@@ -792,6 +804,7 @@ int build_work(pk_ctx *c) {
                             packed[nw + wi] = (int)k0;
                             packed[2 * nw + wi] = (int)std::min(group, koff[t + 1] - k0);
                             packed[3 * nw + wi] = tasks[t].first;
+                            wsteps[wi] = (float)(steps[u] / nc);
                         }
                     }
                 };
@@ -802,40 +815,83 @@ int build_work(pk_ctx *c) {
                 for (size_t t = 0; t < tasks.size(); ++t)
                     if (!whole(t)) fill(t);  // part_of adds records
                 w.nwaves = (int)nw;
-                if (rows) {
-                    // most expensive work items first, so that none of them ends the list
-                    // alone (n-C10H22 / cc-pVTZ: (dd|dp) 5.2 -> 3.4 ms, (fd|dp) 3.1 -> 2.1 ms)
-                    std::vector<double> cost(nw, 0.0);
-                    parallel_for(nw, [&](size_t i) {
-                        const int kb = nprim(packed[i]);
-                        for (int j = 0; j < packed[2 * nw + i]; ++j) cost[i] += 1.0 + kb * nprim(kets[packed[nw + i] + j]);
-                    }, 1024);
-                    std::vector<int> o(nw);
-                    std::iota(o.begin(), o.end(), 0);
-                    std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return cost[x] > cost[y]; });
-                    std::vector<int> q(4 * nw);
-                    for (int k = 0; k < 4; ++k)
-                        for (size_t i = 0; i < nw; ++i) q[k * nw + i] = packed[k * nw + o[i]];
-                    packed.swap(q);
-                }
-                int rc;
-                if ((rc = dev_upload(&w.d_wave, packed, c->stream)) != PK_OK) return rc;
-                if ((rc = dev_upload(&w.d_kets, kets.get(), koff.back(), c->stream)) != PK_OK) return rc;
+                std::vector<int> seg;
                 if (!rows) {
-                    // segments of the per-lane kernels: each bra's waves in runs
-                    // of at most kSegWaves; LDS columns: the two ket shell types
-                    // of the largest molecule
-                    std::vector<int> seg;
+                    // segments of the per-lane kernels: each bra's waves in runs of at
+                    // most segw, shorter where they take more than 1/kSegs of the
+                    // list's steps; LDS columns: the two ket shell types of the largest
+                    // molecule
+                    const size_t segw = std::min<size_t>(kSegWaves, std::max<size_t>(kSegWavesMin, nw / kSegs));
+                    const double seg_most = std::accumulate(tsteps.begin(), tsteps.end(), 0.0) / kSegs;
+                    auto cut = [&](size_t t, auto &&add) {
+                        double sum = 0.0;
+                        for (size_t u = woff[t], n = 0; u < woff[t + 1]; ++u, ++n) {
+                            if (u == woff[t] || n == segw || (n >= kSegWavesMin && sum + wsteps[u] > seg_most)) {
+                                add((int)u);
+                                n = 0;
+                                sum = 0.0;
+                            }
+                            sum += wsteps[u];
+                        }
+                    };
+                    std::vector<size_t> soff(tasks.size() + 1, 0);
+                    parallel_for(tasks.size(), [&](size_t t) { cut(t, [&](int) { ++soff[t + 1]; }); }, grain);
                     for (size_t t = 0; t < tasks.size(); ++t) {
-                        for (size_t w0 = woff[t]; w0 < woff[t + 1]; w0 += kSegWaves) seg.push_back((int)w0);
+                        soff[t + 1] += soff[t];
                         if (woff[t + 1] > woff[t]) {
                             const int *tb = &c->tblk[5 * tasks[t].first];
                             const int ncol = tb[f.lc + 1] - tb[f.lc] + (f.lc == f.ld ? 0 : tb[f.ld + 1] - tb[f.ld]);
                             w.kcols = std::max(w.kcols, ncol);
                         }
                     }
-                    seg.push_back((int)nw);
-                    w.nseg = (int)seg.size() - 1;
+                    w.nseg = (int)soff.back();
+                    seg.resize((size_t)w.nseg + 1, (int)nw);
+                    parallel_for(tasks.size(), [&](size_t t) {
+                        size_t i = soff[t];
+                        cut(t, [&](int u) { seg[i++] = u; });
+                    }, grain);
+                }
+                // Most expensive work first, so that no segment or work item ends the list
+                // alone: segments, to a factor of two (their neighbours share the
+                // bra's densities), and the items of the row kernels.  n-C10H22 / cc-pVTZ,
+                // segments: (ps|ps) 5.4 -> 3.9 ms, (dp|ps) 7.5 -> 6.7, (fp|ps) 4.0 -> 3.2,
+                // (ds|ss) 3.7 -> 3.1; items: (dd|dp) 5.2 -> 3.4, (fd|dp) 3.1 -> 2.1.  The waves
+                // stay in bra order, which plain lists are run in: (ps|ss) 6.7 ms against 7.4
+                // in cost order.
+                if (rows) {
+                    std::vector<double> cost(nw, 0.0);
+                    parallel_for(nw, [&](size_t i) {
+                        const int kb = nprim(packed[i]);
+                        for (int j = 0; j < packed[2 * nw + i]; ++j) cost[i] += 1.0 + (double)kb * nprim(kets[packed[nw + i] + j]);
+                    }, 512);
+                    std::vector<int> o(nw), q(4 * nw);
+                    std::iota(o.begin(), o.end(), 0);
+                    std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+                    for (int k = 0; k < 4; ++k)
+                        for (size_t i = 0; i < nw; ++i) q[k * nw + i] = packed[k * nw + o[i]];
+                    packed.swap(q);
+                } else {
+                    // counting sort by the steps' binary exponent
+                    std::vector<unsigned char> key(w.nseg);
+                    std::array<int, 257> at{};
+                    for (int i = 0; i < w.nseg; ++i) {
+                        float x = 0.f;
+                        for (int u = seg[i]; u < seg[i + 1]; ++u) x += wsteps[u];
+                        ++at[1 + (key[i] = (unsigned char)(255 - std::min(255, std::max(0, std::ilogb(x)))))];
+                    }
+                    std::partial_sum(at.begin(), at.end(), at.begin());
+                    std::vector<int> q(2 * (size_t)w.nseg);
+                    for (int i = 0; i < w.nseg; ++i) {
+                        const size_t n = at[key[i]]++;
+                        q[2 * n] = seg[i];
+                        q[2 * n + 1] = seg[i + 1];
+                    }
+                    seg.swap(q);
+                }
+                int rc;
+                if ((rc = dev_upload(&w.d_wave, packed, c->stream)) != PK_OK) return rc;
+                if ((rc = dev_upload(&w.d_kets, kets.get(), koff.back(), c->stream)) != PK_OK) return rc;
+                if (!rows) {
                     if ((rc = dev_upload(&w.d_seg, seg, c->stream)) != PK_OK) return rc;
                 } else {
                     // LDS columns of the row kernels: the ket's second shell type
@@ -1186,23 +1242,42 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
             const size_t wave_bytes = r.wave_bytes[rk - 1];
             const void *k = uhf ? r.k2 : r.k1;
             // exchange rows of the kets' second shells in LDS, beside at least one
-            // wave; then as many waves as fit, four (two workgroups per CU) at most
+            // wave
             const size_t jrow = (size_t)pk::ncart(f.la) * pk::ncart(f.lb) * sizeof(double);
             size_t krow = (size_t)rk * (pk::ncart(f.la) + pk::ncart(f.lb)) * w.kcols * sizeof(double) + jrow;
             a.segmode = c->seg_on && krow + wave_bytes <= kLdsMax;
             if (!a.segmode) krow = jrow;
-            int waves = w.block > 0 ? w.block / 64 : kDefaultBlock / 64;
-            const int groups = (w.group + r.qw - 1) / r.qw;  // of the largest work item
-            while (waves > 1 && (waves / 2 >= groups || krow + (size_t)waves * wave_bytes > kLdsMax)) waves /= 2;
-            // eight groups per turn of a wave, fewer where the item has fewer
-            a.chunk = std::max(1, std::min(8, groups / (2 * waves)));
-            w.block_run = 64 * waves;
             static std::atomic<int> attr_done[2 * kQuartClasses];  // zero-initialised
             std::atomic<int> &done = attr_done[2 * w.cls + rk - 1];
             if (!done.load()) {
                 PK_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax));
                 done.store(1);
             }
+            const int groups = (w.group + r.qw - 1) / r.qw;  // of the largest work item
+            if (w.row_waves[rk - 1] == 0) {
+                // Waves per workgroup: as few as keep the most waves resident on a CU
+                // (they share the exchange rows in LDS), two at least.  A workgroup's
+                // waves wait for its last one before the flush; n-C10H22 / cc-pVTZ, two
+                // waves against four where both keep eight resident: (dp|pp) 4.3 / 4.8 ms,
+                // (pp|pp) 1.9 / 2.2, (fs|pp) 2.4 / 2.7; six against eight: (fp|dp) 3.0 / 2.5,
+                // (fd|dp) 2.6 / 2.2; one against two (five against eight): (dp|pp) 5.5 / 4.3
+                int best = 0, most = 0;
+                for (int n = kRowWavesMax; n >= 2; n /= 2) {
+                    int wgs = 0;
+                    if (krow + (size_t)n * wave_bytes > kLdsMax) continue;
+                    PK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&wgs, k, 64 * n, krow + (size_t)n * wave_bytes));
+                    if (wgs * n >= most) {
+                        most = wgs * n;
+                        best = n;
+                    }
+                }
+                w.row_waves[rk - 1] = std::max(1, best);
+            }
+            int waves = w.block > 0 ? w.block / 64 : w.row_waves[rk - 1];
+            while (waves > 1 && (waves / 2 >= groups || krow + (size_t)waves * wave_bytes > kLdsMax)) waves /= 2;
+            // eight groups per turn of a wave, fewer where the item has fewer
+            a.chunk = std::max(1, std::min(8, groups / (2 * waves)));
+            w.block_run = 64 * waves;
             int grid = w.nwaves;
             if (w.remap) grid = (grid + 7) / 8 * 8;
             void *args[] = {&a};
@@ -1222,12 +1297,10 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
         const bool alt = seg_alt && a.segmode;  // the segment-mode variant of a plain OS class
         // lanes per workgroup: the autotuned (or PK_BLOCK) shape, else one wave
         // per workgroup for the segment-mode lists of a batch of molecules whose
-        // exchange rows leave room for at least 6 such workgroups per CU, and
-        // kDefaultBlock otherwise.  Measured per class list: on the 256 water
-        // clusters (rows of 2-19 KB) every list is faster with one wave (batched
-        // build 356 -> 256 ms); on n-C10H22 / cc-pVTZ (one molecule, segments of
-        // many kets) most lists are faster with four ((pp|ss) 7.4 -> 3.5 ms,
-        // (dd|dp) 11.4 -> 7.4 ms; a few lose up to 0.8 ms)
+        // exchange rows leave room for at least 6 such workgroups per CU (256 water
+        // clusters, rows of 2-19 KB: every list is faster with one wave, 356 -> 256 ms
+        // for the build), and kDefaultBlock otherwise (one molecule, segments of
+        // many kets: n-C10H22 / cc-pVTZ (pp|ss) 7.4 -> 3.5 ms with four waves for one)
         const bool one_wave =
             a.segmode && c->nmol > 1 && pk::jk_lds_bytes(a, f.la, f.lb, nk) <= kSegOneWaveLds;
         const int block = w.block > 0 ? w.block : (one_wave ? 64 : kDefaultBlock);

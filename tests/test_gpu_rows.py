@@ -82,3 +82,28 @@ def test_short_build_in_one_launch_equals_its_lists(mol, basis):
         # prepare, s/p/d lists, f lists, finalize, and the five classes outside the
         # launch: (fd|ss), (ff|ss), (fd|fd), (ff|fd), (ff|ff)
         assert eng.stats()["kernel_launches"] <= 9
+
+
+@pytest.mark.parametrize("engine", ["os", "rys"])
+@pytest.mark.parametrize("alt", ["0", "1000"])
+def test_segments_equal_plain_lists(engine, alt, monkeypatch):
+    """Lists of more than 256 segments (n-C8H18 / cc-pVDZ, its waves too many for
+    a short build): segments cut by steps and run most expensive first, workgroups
+    of the row kernels by residency, against the same lists without exchange rows.
+    Same integrals, another order of at most 1e6 FP64 sums: 1e-11 of the largest
+    element."""
+    Z, X = alkane(8)
+    from pkfock.host import Molecule
+
+    shells = Molecule(Z, X, "cc-pvdz").shells()
+    out = []
+    for rows in ("1", "0"):
+        monkeypatch.setenv("PK_EXCHANGE_ROWS", rows)
+        monkeypatch.setenv("PK_SEG_ALT_PRIM", alt)
+        eng = FockEngine(shells, engine, 1e-11)
+        rng = np.random.default_rng(24)
+        A, B = rng.normal(size=(2, eng.nbasis, eng.nbasis)) * 0.2
+        out.append(eng.jk(A + A.T) + eng.jk_uhf(A + A.T, B + B.T))
+        eng.close()
+    for x, y in zip(*out):
+        assert np.abs(x - y).max() < 1e-11 * np.abs(y).max()
