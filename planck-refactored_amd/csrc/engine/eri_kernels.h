@@ -409,9 +409,25 @@ __device__ __forceinline__ void jk_run(const JKArgs &a, int w_first, int w_end, 
     }
 }
 
+// Waves per SIMD that the FP64 kernel is compiled for: two where the registers
+// above 256 are few enough that spilling them costs less than a second wave
+// gives (one wave cannot hide the latency of the Boys and Rys gathers: (dp|ps)
+// keeps the vector unit busy 23 % of the time).  Measured on n-C10H22 / cc-pVTZ, one wave ->
+// two: Obara-Saika (ds|ds) 2.9 -> 1.9 ms, (fp|ss) 1.31 -> 0.87, (dd|ss) 1.23 -> 1.08, but
+// (dp|ps), 48 accumulators, 6.7 -> 7.5 and (ds|pp), 54, 5.2 -> 5.8; Rys (dp|ds) 8.0 -> 6.3,
+// (fs|ds) 2.9 -> 2.6, but bras of higher order (dd|ps) 4.1 -> 6.3, (fp|ps) 3.2 -> 6.9.
+// Rys kernels of fewer accumulators fit 256 registers by themselves, and the bound
+// costs them up to 9 % ((fs|ps) 2.7 -> 3.0).
+constexpr int jk_min_waves(int la, int lb, int lc, int ld, int alg, int ncomp) {
+    const int ne = nlev(la, la + lb);
+    if (alg == ALG_OS) return ne * nlev(lc, lc + ld) <= 40 ? 2 : 1;
+    return la + lb <= 3 && ne * ncomp >= 48 ? 2 : 1;
+}
+
 // SEGV: 1 / 0 compiles the segment-mode / plain kernel, -1 takes seg_class.
 template <typename R, int LA, int LB, int LC, int LD, int ALG, int C0, int C1, int NK = 1, int SEGV = -1>
-__global__ __launch_bounds__(256) void k_jk(JKArgs a) {
+__global__ __launch_bounds__(256, (std::is_same_v<R, double> && NK == 1 ? jk_min_waves(LA, LB, LC, LD, ALG, C1 - C0) : 1)) void k_jk(
+    JKArgs a) {
     extern __shared__ double krow[];
     constexpr bool SEG = SEGV >= 0 ? SEGV != 0 : seg_class(LA, LB, LC, LD);
     int w_first, w_end, w_step, w_lead;
