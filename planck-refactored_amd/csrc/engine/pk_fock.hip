@@ -620,16 +620,24 @@ int build_work(pk_ctx *c) {
     // records of parts of pairs (primitives [p0, p1)), indexed after the pairs
     std::vector<pk::PairDev> vpairs;
     std::unordered_map<uint64_t, int> vindex;
+    std::vector<int> npr(np);  // primitive counts beside the records (one per quartet is read)
+    for (int p = 0; p < np; ++p) npr[p] = c->pairs[p].nprim;
+    std::vector<double> steps;  // steps of the list's waves before the cuts (kept from list to list: page faults)
+    std::vector<float> wsteps;  // and after them
+    std::vector<int> part_base;  // first of a ket's parts, of the list at hand
+    auto add_part = [&](int p, int p0, int p1) {
+        pk::PairDev v = c->pairs[p];
+        v.prim_off += p0;
+        v.nprim = p1 - p0;
+        vpairs.push_back(v);
+        return np + (int)vpairs.size() - 1;
+    };
     auto part_of = [&](int p, int p0, int p1) {
         if (p1 - p0 >= c->pairs[p].nprim) return p;
         const uint64_t key = ((uint64_t)p << 24) | ((uint64_t)p0 << 12) | (uint64_t)p1;  // nprim < 2048
         const auto it = vindex.find(key);
         if (it != vindex.end()) return it->second;
-        pk::PairDev v = c->pairs[p];
-        v.prim_off += p0;
-        v.nprim = p1 - p0;
-        vpairs.push_back(v);
-        return vindex[key] = np + (int)vpairs.size() - 1;
+        return vindex[key] = add_part(p, p0, p1);
     };
     struct BraRange {
         size_t k0 = 0, k1 = 0;  // positions [k0, k1) of the q-ordered kets
@@ -728,12 +736,12 @@ int build_work(pk_ctx *c) {
                         for (size_t i = 0; i < n; ++i) dst[i] = kk[i].second;
                     }
                     const int b = by_cls[m][cb][tasks[t].second];
-                    const int kb = c->pairs[b].nprim;
-                    for (size_t i = 0; i < n; ++i) {
-                        const double K = (double)kb * c->pairs[dst[i]].nprim;
-                        o.nprimq += (int64_t)K;
-                        o.flops += pk::model_flops(f.la, f.lb, f.lc, f.ld, K);
-                    }
+                    int64_t nk = 0;
+                    for (size_t i = 0; i < n; ++i) nk += npr[dst[i]];
+                    o.nprimq = npr[b] * nk;
+                    // the model is linear in the primitive quartets of a quartet
+                    const double f0 = pk::model_flops(f.la, f.lb, f.lc, f.ld, 0.0);
+                    o.flops = (double)n * f0 + (double)o.nprimq * (pk::model_flops(f.la, f.lb, f.lc, f.ld, 1.0) - f0);
                 });
                 for (size_t t = 0; t < tasks.size(); ++t) {
                     w.nquart += (int64_t)(outs[t].k1 - outs[t].k0);
@@ -754,10 +762,21 @@ int build_work(pk_ctx *c) {
                     // few quartets for the chip: every ket as its parts, neighbours
                     std::vector<int> ex;
                     std::vector<size_t> off(1, 0);
+                    ex.reserve(koff.back() * parts);
+                    part_base.assign(np, -1);
                     for (size_t t = 0; t < tasks.size(); ++t) {
                         for (size_t k = koff[t]; k < koff[t + 1]; ++k) {
                             const int nk = c->pairs[kets[k]].nprim, m = std::max(1, std::min((int)parts, nk));
-                            for (int i = 0; i < m; ++i) ex.push_back(part_of(kets[k], nk * i / m, nk * (i + 1) / m));
+                            if (m == 1) {
+                                ex.push_back(kets[k]);
+                                continue;
+                            }
+                            int &b0 = part_base[kets[k]];  // the pair's m parts, neighbours
+                            if (b0 < 0) {
+                                b0 = np + (int)vpairs.size();
+                                for (int i = 0; i < m; ++i) add_part(kets[k], nk * i / m, nk * (i + 1) / m);
+                            }
+                            for (int i = 0; i < m; ++i) ex.push_back(b0 + i);
                         }
                         off.push_back(ex.size());
                     }
@@ -766,11 +785,14 @@ int build_work(pk_ctx *c) {
                     std::copy(ex.begin(), ex.end(), kets.get());
                     koff.swap(off);
                 }
-                auto nprim = [&](int p) { return p < np ? c->pairs[p].nprim : vpairs[p - np].nprim; };
+                auto nprim = [&](int p) { return p < np ? npr[p] : vpairs[p - np].nprim; };
                 std::vector<size_t> uoff(tasks.size() + 1, 0), woff(tasks.size() + 1, 0);  // waves before and after
                 for (size_t t = 0; t < tasks.size(); ++t) uoff[t + 1] = uoff[t] + (koff[t + 1] - koff[t] + group - 1) / group;
-                const size_t grain = uoff.back() > 65536 ? 64 : 4096;
-                std::vector<double> steps(uoff.back()), tsteps(tasks.size(), 0.0);
+                // a thread per 32768 waves (one takes about 0.1 ms for them, and tens of
+                // microseconds to start)
+                const size_t grain = std::max<size_t>(64, tasks.size() * 32768 / std::max<size_t>(1, uoff.back()));
+                std::vector<double> tsteps(tasks.size(), 0.0), tmost(tasks.size(), 0.0);  // a bra's steps, its longest wave
+                if (steps.size() < uoff.back()) steps.resize(uoff.back());
                 auto bra_of = [&](size_t t) { return by_cls[tasks[t].first][cb][tasks[t].second]; };
                 parallel_for(tasks.size(), [&](size_t t) {
                     const int kb = c->pairs[bra_of(t)].nprim;
@@ -778,21 +800,29 @@ int build_work(pk_ctx *c) {
                         const size_t k0 = koff[t] + (u - uoff[t]) * group, m = std::min(group, koff[t + 1] - k0);
                         steps[u] = (double)kb * nprim(kets[k0]) * ((m + per - 1) / per);
                         tsteps[t] += steps[u];
+                        tmost[t] = std::max(tmost[t], steps[u]);
                     }
                 }, grain);
                 const double most = std::max(kCutSteps, std::accumulate(tsteps.begin(), tsteps.end(), 0.0) /
                                                             (rows ? kRowItems / 4 : kCutWaves));
                 auto cuts = [&](int kb, size_t u) { return std::max(1, std::min(kb, (int)(steps[u] / most))); };
-                parallel_for(tasks.size(), [&](size_t t) {
-                    const int kb = c->pairs[bra_of(t)].nprim;
-                    size_t n = 0;
-                    for (size_t u = uoff[t]; u < uoff[t + 1]; ++u) n += cuts(kb, u);
-                    woff[t + 1] = n;
-                }, grain);
-                for (size_t t = 0; t < tasks.size(); ++t) woff[t + 1] += woff[t];
+                if (*std::max_element(tmost.begin(), tmost.end()) < 2.0 * most) {
+                    woff = uoff;  // no wave is cut
+                } else {
+                    parallel_for(tasks.size(), [&](size_t t) {
+                        const int kb = c->pairs[bra_of(t)].nprim;
+                        size_t n = uoff[t + 1] - uoff[t];
+                        if (tmost[t] >= 2.0 * most) {
+                            n = 0;
+                            for (size_t u = uoff[t]; u < uoff[t + 1]; ++u) n += cuts(kb, u);
+                        }
+                        woff[t + 1] = n;
+                    }, grain);
+                    for (size_t t = 0; t < tasks.size(); ++t) woff[t + 1] += woff[t];
+                }
                 const size_t nw = woff.back();
                 std::vector<int> packed(4 * nw);
-                std::vector<float> wsteps(nw);  // steps of every wave
+                if (wsteps.size() < nw) wsteps.resize(nw);
                 auto fill = [&](size_t t) {
                     const int b = bra_of(t), kb = c->pairs[b].nprim;
                     size_t wi = woff[t];
