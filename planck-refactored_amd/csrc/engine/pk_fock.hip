@@ -288,8 +288,12 @@ __global__ void k_finalize(const double *__restrict__ A, const double *__restric
     if (G) G[o + i] = j - 0.5 * k;
 }
 
+// Autotuned launch shape of a class list.  A class of pk::small_rows runs its short
+// lists in another kernel than its long ones, so a choice holds for lists of its kind.
 struct TuneEntry {
-    int cls, prec, block, remap, alt;
+    int cls, prec;
+    bool rows;
+    int block, remap, alt;
 };
 
 struct ClassWork {
@@ -298,8 +302,8 @@ struct ClassWork {
     int block = 0;            // lanes per workgroup (autotuned or PK_BLOCK; 0: the default of the launch)
     int block_run = 0;        // lanes per workgroup of the last launch
     int remap = 0;            // XCD-contiguous wave ranges (autotuned)
-    int alt = 0;              // alternative kernel (autotuned): FP64 integrals for an FP32 list,
-                              // the cooperative kernel for a per-lane Rys class
+    int alt = 0;              // alternative kernel (autotuned, see has_alt): FP64 integrals for an
+                              // FP32 list, the cooperative kernel for a per-lane Rys list
     int nwaves = 0;
     int64_t nquart = 0;
     int64_t nprimq = 0;
@@ -431,6 +435,11 @@ int list_kind(const pk_ctx *c, const ClassWork &w) {
     if (use_os(c, f)) return fp32 ? 3 : 0;
     if (!w.rows && !(w.alt && w.prec == PK_PREC_FP64)) return fp32 ? 4 : 1;
     return 2;
+}
+
+// lists with an alternative kernel (ClassWork::alt)
+bool has_alt(const pk_ctx *c, const ClassWork &w) {
+    return w.prec == PK_PREC_MIXED || (!w.rows && !use_os(c, kClasses[w.cls]));
 }
 
 // lists that k_small takes: Obara-Saika classes and rows (in FP64)
@@ -948,7 +957,7 @@ int build_work(pk_ctx *c) {
     // launch shapes chosen by pk_ctx_autotune for this context, if any
     for (ClassWork &w : c->work)
         for (const TuneEntry &t : c->tuned)
-            if (t.cls == w.cls && t.prec == w.prec) {
+            if (t.cls == w.cls && t.prec == w.prec && t.rows == w.rows) {
                 w.block = t.block;
                 w.remap = t.remap;
                 w.alt = t.alt;
@@ -1836,7 +1845,7 @@ int pk_ctx_autotune(pk_ctx *c, int reps) {
         for (ClassWork &w : c->work) {
             w.block = cand[k][0];
             w.remap = cand[k][1];
-            w.alt = cand[k][2];
+            w.alt = cand[k][2] && has_alt(c, w);
         }
         std::vector<double> t(nw, 0.0);
         for (int r = 0; r < nrep; ++r) {
@@ -1851,7 +1860,7 @@ int pk_ctx_autotune(pk_ctx *c, int reps) {
         }
         if (keep)
             for (size_t i = 0; i < nw; ++i)
-                if (t[i] < best[i]) {
+                if (t[i] < best[i] && c->work[i].alt == cand[k][2]) {
                     best[i] = t[i];
                     pick[i] = k;
                 }
@@ -1869,7 +1878,7 @@ int pk_ctx_autotune(pk_ctx *c, int reps) {
         w.alt = cand[pick[i]][2];
         w.ms_total = 0.0;
         w.builds = 0;
-        c->tuned.push_back(TuneEntry{w.cls, w.prec, w.block, w.remap, w.alt});
+        c->tuned.push_back(TuneEntry{w.cls, w.prec, w.rows, w.block, w.remap, w.alt});
     }
     drop_graph(c);
     return PK_OK;
