@@ -109,8 +109,10 @@ int pk_ctx_set_graph(pk_ctx *ctx, int enable);
  * (1, 2 or 4 waves per workgroup; with or without XCD-contiguous wave ranges;
  * the list's alternative kernel: FP64 integrals for an FP32 list of the mixed
  * precision, the cooperative kernel for a class with per-lane Rys kernels)
- * over `reps` builds and keeps the fastest per class for this context.  The
- * density buffer is overwritten. */
+ * over `reps` builds and keeps the fastest per class for this context; a build
+ * short enough for one launch takes its lists so tuned or the one launch,
+ * whichever is faster.  The choices outlive a change of the work lists
+ * (pk_ctx_set).  The density buffer is overwritten. */
 int pk_ctx_autotune(pk_ctx *ctx, int reps);
 
 /* Engine and threshold (types.h:407-411).  precision PK_PREC_MIXED computes

@@ -397,6 +397,7 @@ struct pk_ctx {
     pk::SmallTab small_tab[2];
     int small_blocks[2] = {0, 0};
     size_t small_lds[2] = {0, 0};
+    bool lists_win = false;  // the tuned lists of a short build beat its one launch (pk_ctx_autotune)
     std::vector<GradWork> gwork;  // gradient work items, built by the first gradient at a tolerance
     int *d_gorder = nullptr;
     double gwork_tol = -1.0;
@@ -446,6 +447,13 @@ bool has_alt(const pk_ctx *c, const ClassWork &w) {
 bool small_covers(const ClassWork &w) {
     const ClassFns &f = kClasses[w.cls];
     return f.small_set >= 0 && (w.rows || f.has_os) && w.prec == PK_PREC_FP64;
+}
+
+// The build goes out in one launch (k_small): a short one whose tuned lists, if any,
+// are not the faster.  k_small holds the FP64 Obara-Saika and row kernels of one
+// exchange density; UHF, mixed precision and the Rys engine run their lists.
+bool one_launch(const pk_ctx *c, const double *B2) {
+    return c->d_small && !c->lists_win && c->engine != PK_ENGINE_RYS && !B2;
 }
 
 void drop_graph(pk_ctx *c) {
@@ -966,7 +974,7 @@ int build_work(pk_ctx *c) {
     int64_t waves = 0;
     for (const ClassWork &w : c->work) waves += w.nwaves;
     std::vector<pk::SmallList> small;  // uploaded from here until the synchronisation below
-    if (waves <= kSmallWaves && !mixed && c->tuned.empty() && !c->block_forced) {
+    if (waves <= kSmallWaves && !mixed && !c->block_forced) {
         c->small_tab[0].n = c->small_tab[1].n = 0;
         c->small_blocks[0] = c->small_blocks[1] = 0;
         c->small_lds[0] = c->small_lds[1] = 0;
@@ -1201,7 +1209,7 @@ int launch_small(pk_ctx *c, const BuildBufs &sb, int &nl) {
 int launch_classes(pk_ctx *c, const BuildBufs &sb, bool events, int &nl) {
     int rc;
     hipStream_t s = c->stream;
-    if (!events && c->d_small && c->engine != PK_ENGINE_RYS && !sb.B2) return launch_small(c, sb, nl);
+    if (!events && one_launch(c, sb.B2)) return launch_small(c, sb, nl);
     // Concurrent queues (not while profiling: the class events time one list
     // at a time): lists in descending model cost, each to the queue with the
     // least cost so far, so that the small classes fill the tails of the
@@ -1822,7 +1830,8 @@ int pk_ctx_mol_layout(const pk_ctx *c, int32_t *nb, int64_t *offset) {
 // Launch-shape autotuner: every class list is timed (HIP events, `reps` builds
 // per candidate after one untimed build) under each candidate shape --
 // workgroups of 1, 2 or 4 waves, with and without XCD-contiguous wave ranges
-// -- and keeps the fastest; the choice persists for the context and is
+// -- and keeps the fastest; a short build then takes its lists so tuned or the one
+// launch, whichever is faster.  The choices persist for the context and are
 // re-applied when the work lists are rebuilt.
 int pk_ctx_autotune(pk_ctx *c, int reps) {
     if (!c) return fail(PK_ERR_ARG, "pk_ctx_autotune: null context");
@@ -1881,6 +1890,28 @@ int pk_ctx_autotune(pk_ctx *c, int reps) {
         c->tuned.push_back(TuneEntry{w.cls, w.prec, w.rows, w.block, w.remap, w.alt});
     }
     drop_graph(c);
+    // a short build: its lists as tuned against the one launch for all of them
+    if (c->d_small && c->engine != PK_ENGINE_RYS) {
+        float ms[2] = {0.f, 0.f};
+        auto time_build = [&](float &t) -> int {
+            PK_HIP(hipEventRecord(c->ev0, s));
+            int rc2;
+            if ((rc2 = launch_build(c, c->d_P, c->d_J, c->d_K, nullptr, ctx_bufs(c), false)) != PK_OK) return rc2;
+            PK_HIP(hipEventRecord(c->ev1, s));
+            PK_HIP(hipEventSynchronize(c->ev1));
+            PK_HIP(hipEventElapsedTime(&t, c->ev0, c->ev1));
+            return PK_OK;
+        };
+        for (int r = 0; r <= reps && rc == PK_OK; ++r)  // the first of each untimed
+            for (int lists = 0; lists < 2 && rc == PK_OK; ++lists) {
+                c->lists_win = lists != 0;
+                float t = 0.f;
+                rc = time_build(t);
+                if (r > 0) ms[lists] += t;
+            }
+        c->lists_win = rc == PK_OK && ms[1] < ms[0];
+        if (rc != PK_OK) return rc;
+    }
     return PK_OK;
 }
 

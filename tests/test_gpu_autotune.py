@@ -52,3 +52,30 @@ def test_tuned_shapes_of_a_long_build():
     for _ in range(3):
         assert _same(eng.jk(P), ref)
     assert _same(got, ref)
+
+
+def _in_one_launch(eng):
+    # prepare, s/p/d lists, f lists, finalize, and at most five classes outside
+    return eng.stats()["kernel_launches"] <= 9 < len(eng.class_stats())
+
+
+@pytest.mark.parametrize("basis", ["6-31g*", "cc-pvtz"])
+def test_short_build_after_autotuning(basis):
+    """The tuner takes the one launch of a short build or its tuned lists; the choice
+    holds before and after the lists are built again, and both give the same."""
+    eng = FockEngine(Molecule(*water(), basis).shells(), "os", 1e-12)
+    P = _density(eng.nbasis, 3)
+    ref = eng.jk(P)
+    assert _in_one_launch(eng)
+    eng.autotune(reps=3)
+    assert _same(eng.jk(P), ref)
+    one = _in_one_launch(eng)
+    eng.profile(True)  # the lists, as tuned
+    assert _same(eng.jk(P), ref) and not _in_one_launch(eng)
+    eng.profile(False)
+    eng.set("os", 0.99e-12)
+    got = eng.jk(P)
+    assert _in_one_launch(eng) == one
+    eng.set("os", 1e-12)
+    assert _same(eng.jk(P), ref) and _in_one_launch(eng) == one
+    assert all(np.abs(x - y).max() < 1e-9 for x, y in zip(got, ref))
