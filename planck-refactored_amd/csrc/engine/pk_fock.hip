@@ -1463,9 +1463,9 @@ int build_device(pk_ctx *c, const double *dP, double *dJ, double *dK, double *dG
     if ((rc = ensure_buffers(c)) != PK_OK) return rc;
     hipStream_t s = c->stream;
     const size_t bytes = c->n2 * sizeof(double);
-    // the first build that would use the side queues times every list (one
-    // at a time), so that later builds balance the queues by measured cost
-    c->learning = !c->cost_learned && !c->profile && c->side_ok && !c->side_off &&
+    // the first build that would spread its lists over the side queues times every
+    // list (one at a time), so that later builds balance the queues by measured cost
+    c->learning = !c->cost_learned && !c->profile && c->side_ok && !c->side_off && !one_launch(c, nullptr) &&
                   c->st.quartets >= kSideMinQuartets && c->work.size() > 1;
     if (!c->graph_on || c->profile || c->learning) {
         PK_HIP(hipEventRecord(c->ev0, s));
