@@ -639,8 +639,23 @@ int build_work(pk_ctx *c) {
     std::unordered_map<uint64_t, int> vindex;
     std::vector<int> npr(np);  // primitive counts beside the records (one per quartet is read)
     for (int p = 0; p < np; ++p) npr[p] = c->pairs[p].nprim;
-    std::vector<double> steps;  // steps of the list's waves before the cuts (kept from list to list: page faults)
-    std::vector<float> wsteps;  // and after them
+    // arrays of the list at hand, kept from list to list (page faults; an upload from
+    // pageable memory has read its source when it returns): the kets,
+    // one index per quartet, not value-initialised (up to GBs for large batches);
+    // the steps of its waves before the cuts, and their primitive pairs (row kernels);
+    // after the cuts the steps of its waves, or the costs of its row items; the first
+    // wave and the order of its segments
+    std::unique_ptr<int[]> kets;
+    size_t kets_cap = 0;
+    auto need_kets = [&](size_t n) {
+        if (n <= kets_cap) return;
+        kets.reset();
+        kets.reset(new int[n]);
+        kets_cap = n;
+    };
+    std::vector<double> steps, ksum, wsteps;
+    std::vector<int> cut_at;
+    std::vector<unsigned char> cut_key;
     std::vector<int> part_base;  // first of a ket's parts, of the list at hand
     auto add_part = [&](int p, int p0, int p1) {
         pk::PairDev v = c->pairs[p];
@@ -726,12 +741,46 @@ int build_work(pk_ctx *c) {
                 std::vector<size_t> koff(tasks.size() + 1, 0);
                 for (size_t t = 0; t < tasks.size(); ++t) koff[t + 1] = koff[t] + (outs[t].k1 - outs[t].k0);
                 if (koff.back() > (size_t)INT32_MAX) return fail(PK_ERR_ARG, "build_work: more than 2^31 quartets in one class");
-                // the ket array is written entirely below: no value-initialisation
-                // (it holds one index per quartet, up to GBs for large batches)
-                std::unique_ptr<int[]> kets(new int[std::max<size_t>(1, koff.back())]);
+                need_kets(koff.back());
+                auto nprim = [&](int p) { return p < np ? npr[p] : vpairs[p - np].nprim; };
+                auto bra_of = [&](size_t t) { return by_cls[tasks[t].first][cb][tasks[t].second]; };
+                // waves of up to `group` kets before the cuts, a bra's steps, its longest
+                // wave.  Steps of a wave: the primitive quartets of its first ket (the
+                // longest within the ordering ratio), per group of slots.
+                const size_t per = rows ? (size_t)rows_table()[cls].qw : 64;
+                std::vector<size_t> uoff(tasks.size() + 1, 0);
+                std::vector<double> tsteps(tasks.size()), tmost(tasks.size());
+                auto count_waves = [&]() {
+                    for (size_t t = 0; t < tasks.size(); ++t)
+                        uoff[t + 1] = uoff[t] + (koff[t + 1] - koff[t] + group - 1) / group;
+                    if (steps.size() < uoff.back()) steps.resize(uoff.back());
+                    if (rows && ksum.size() < uoff.back()) ksum.resize(uoff.back());
+                };
+                auto count_steps = [&](size_t t) {
+                    const int kb = npr[bra_of(t)];
+                    double sum = 0.0, most = 0.0;
+                    for (size_t u = uoff[t]; u < uoff[t + 1]; ++u) {
+                        const size_t k0 = koff[t] + (u - uoff[t]) * group, m = std::min(group, koff[t + 1] - k0);
+                        steps[u] = (double)kb * nprim(kets[k0]) * ((m + per - 1) / per);
+                        sum += steps[u];
+                        most = std::max(most, steps[u]);
+                        if (rows) {
+                            int64_t nk = 0;
+                            for (size_t k = k0; k < k0 + m; ++k) nk += nprim(kets[k]);
+                            ksum[u] = (double)nk;
+                        }
+                    }
+                    tsteps[t] = sum;
+                    tmost[t] = most;
+                };
+                count_waves();
+                // quartets that fill the chip; a list of at most half as many may have its
+                // kets cut below, and its steps are counted after that
+                const size_t fill_quart = rows ? kSplitSlots * per : kSplitLanes;
+                const bool few = 2 * koff.back() <= fill_quart;
                 // pass 2: every bra's kets in ket order (ordering group
                 // descending, then first and second function) straight into the
-                // flat array, and its waves
+                // flat array, and, while they are in the cache, the steps of its waves
                 parallel_for(tasks.size(), [&](size_t t) {
                     BraRange &o = outs[t];
                     const size_t n = o.k1 - o.k0;
@@ -752,10 +801,10 @@ int build_work(pk_ctx *c) {
                         std::sort(kk.begin(), kk.end());
                         for (size_t i = 0; i < n; ++i) dst[i] = kk[i].second;
                     }
-                    const int b = by_cls[m][cb][tasks[t].second];
                     int64_t nk = 0;
                     for (size_t i = 0; i < n; ++i) nk += npr[dst[i]];
-                    o.nprimq = npr[b] * nk;
+                    o.nprimq = npr[bra_of(t)] * nk;
+                    if (!few) count_steps(t);
                     // the model is linear in the primitive quartets of a quartet
                     const double f0 = pk::model_flops(f.la, f.lb, f.lc, f.ld, 0.0);
                     o.flops = (double)n * f0 + (double)o.nprimq * (pk::model_flops(f.la, f.lb, f.lc, f.ld, 1.0) - f0);
@@ -766,15 +815,10 @@ int build_work(pk_ctx *c) {
                     w.flops += outs[t].flops;
                 }
                 if (w.nquart == 0) continue;
-                // Waves of up to `group` kets, cut along the bra's primitives where a
-                // wave would take more than about 1/kCutWaves of the list's steps.  Steps
-                // of a wave: the primitive quartets of its first ket (the longest within
-                // the ordering ratio), per group of slots.
-                const size_t per = rows ? (size_t)rows_table()[cls].qw : 64;
                 const size_t parts =
                     w.nprimq < (int64_t)kSplitPrims * w.nquart
                         ? 1
-                        : std::min<size_t>(kSplitMost, (rows ? kSplitSlots * per : kSplitLanes) / (size_t)w.nquart);
+                        : std::min<size_t>(kSplitMost, fill_quart / (size_t)w.nquart);
                 if (parts > 1) {
                     // few quartets for the chip: every ket as its parts, neighbours
                     std::vector<int> ex;
@@ -798,28 +842,18 @@ int build_work(pk_ctx *c) {
                         off.push_back(ex.size());
                     }
                     if (ex.size() > (size_t)INT32_MAX) return fail(PK_ERR_ARG, "build_work: more than 2^31 quartets in one class");
-                    kets.reset(new int[ex.size()]);
+                    need_kets(ex.size());
                     std::copy(ex.begin(), ex.end(), kets.get());
                     koff.swap(off);
+                    count_waves();
                 }
-                auto nprim = [&](int p) { return p < np ? npr[p] : vpairs[p - np].nprim; };
-                std::vector<size_t> uoff(tasks.size() + 1, 0), woff(tasks.size() + 1, 0);  // waves before and after
-                for (size_t t = 0; t < tasks.size(); ++t) uoff[t + 1] = uoff[t] + (koff[t + 1] - koff[t] + group - 1) / group;
                 // a thread per 32768 waves (one takes about 0.1 ms for them, and tens of
                 // microseconds to start)
                 const size_t grain = std::max<size_t>(64, tasks.size() * 32768 / std::max<size_t>(1, uoff.back()));
-                std::vector<double> tsteps(tasks.size(), 0.0), tmost(tasks.size(), 0.0);  // a bra's steps, its longest wave
-                if (steps.size() < uoff.back()) steps.resize(uoff.back());
-                auto bra_of = [&](size_t t) { return by_cls[tasks[t].first][cb][tasks[t].second]; };
-                parallel_for(tasks.size(), [&](size_t t) {
-                    const int kb = c->pairs[bra_of(t)].nprim;
-                    for (size_t u = uoff[t]; u < uoff[t + 1]; ++u) {
-                        const size_t k0 = koff[t] + (u - uoff[t]) * group, m = std::min(group, koff[t + 1] - k0);
-                        steps[u] = (double)kb * nprim(kets[k0]) * ((m + per - 1) / per);
-                        tsteps[t] += steps[u];
-                        tmost[t] = std::max(tmost[t], steps[u]);
-                    }
-                }, grain);
+                if (few) parallel_for(tasks.size(), count_steps, grain);
+                // Waves are cut along the bra's primitives where one would take more than
+                // about 1/kCutWaves of the list's steps.
+                std::vector<size_t> woff(tasks.size() + 1, 0);
                 const double most = std::max(kCutSteps, std::accumulate(tsteps.begin(), tsteps.end(), 0.0) /
                                                             (rows ? kRowItems / 4 : kCutWaves));
                 auto cuts = [&](int kb, size_t u) { return std::max(1, std::min(kb, (int)(steps[u] / most))); };
@@ -851,7 +885,7 @@ int build_work(pk_ctx *c) {
                             packed[nw + wi] = (int)k0;
                             packed[2 * nw + wi] = (int)std::min(group, koff[t + 1] - k0);
                             packed[3 * nw + wi] = tasks[t].first;
-                            wsteps[wi] = (float)(steps[u] / nc);
+                            wsteps[wi] = rows ? packed[2 * nw + wi] + (double)nprim(packed[wi]) * ksum[u] : steps[u] / nc;
                         }
                     }
                 };
@@ -867,36 +901,50 @@ int build_work(pk_ctx *c) {
                     // segments of the per-lane kernels: each bra's waves in runs of at
                     // most segw, shorter where they take more than 1/kSegs of the
                     // list's steps; LDS columns: the two ket shell types of the largest
-                    // molecule
+                    // molecule.  The segments of bra task t from woff[t] on.
                     const size_t segw = std::min<size_t>(kSegWaves, std::max<size_t>(kSegWavesMin, nw / kSegs));
                     const double seg_most = std::accumulate(tsteps.begin(), tsteps.end(), 0.0) / kSegs;
-                    auto cut = [&](size_t t, auto &&add) {
+                    if (cut_at.size() < nw) cut_at.resize(nw), cut_key.resize(nw);
+                    std::vector<int> nseg(tasks.size(), 0);
+                    parallel_for(tasks.size(), [&](size_t t) {
+                        size_t i = woff[t], n = 0;
                         double sum = 0.0;
-                        for (size_t u = woff[t], n = 0; u < woff[t + 1]; ++u, ++n) {
+                        // order among the segments: the steps' binary exponent, descending
+                        auto close = [&]() {
+                            if (i > woff[t]) cut_key[i - 1] = (unsigned char)(255 - std::min(255, std::max(0, std::ilogb(sum))));
+                        };
+                        for (size_t u = woff[t]; u < woff[t + 1]; ++u, ++n) {
                             if (u == woff[t] || n == segw || (n >= kSegWavesMin && sum + wsteps[u] > seg_most)) {
-                                add((int)u);
+                                close();
+                                cut_at[i++] = (int)u;
                                 n = 0;
                                 sum = 0.0;
                             }
                             sum += wsteps[u];
                         }
-                    };
-                    std::vector<size_t> soff(tasks.size() + 1, 0);
-                    parallel_for(tasks.size(), [&](size_t t) { cut(t, [&](int) { ++soff[t + 1]; }); }, grain);
+                        close();
+                        nseg[t] = (int)(i - woff[t]);
+                    }, grain);
                     for (size_t t = 0; t < tasks.size(); ++t) {
-                        soff[t + 1] += soff[t];
+                        w.nseg += nseg[t];
                         if (woff[t + 1] > woff[t]) {
                             const int *tb = &c->tblk[5 * tasks[t].first];
                             const int ncol = tb[f.lc + 1] - tb[f.lc] + (f.lc == f.ld ? 0 : tb[f.ld + 1] - tb[f.ld]);
                             w.kcols = std::max(w.kcols, ncol);
                         }
                     }
-                    w.nseg = (int)soff.back();
-                    seg.resize((size_t)w.nseg + 1, (int)nw);
-                    parallel_for(tasks.size(), [&](size_t t) {
-                        size_t i = soff[t];
-                        cut(t, [&](int u) { seg[i++] = u; });
-                    }, grain);
+                    // counting sort
+                    std::array<int, 257> at{};
+                    for (size_t t = 0; t < tasks.size(); ++t)
+                        for (int i = 0; i < nseg[t]; ++i) ++at[1 + cut_key[woff[t] + i]];
+                    std::partial_sum(at.begin(), at.end(), at.begin());
+                    seg.resize(2 * (size_t)w.nseg);
+                    for (size_t t = 0; t < tasks.size(); ++t)
+                        for (int i = 0; i < nseg[t]; ++i) {
+                            const size_t n = at[cut_key[woff[t] + i]]++;
+                            seg[2 * n] = cut_at[woff[t] + i];
+                            seg[2 * n + 1] = i + 1 < nseg[t] ? cut_at[woff[t] + i + 1] : (int)woff[t + 1];
+                        }
                 }
                 // Most expensive work first, so that no segment or work item ends the list
                 // alone: segments, to a factor of two (their neighbours share the
@@ -906,34 +954,12 @@ int build_work(pk_ctx *c) {
                 // stay in bra order, which plain lists are run in: (ps|ss) 6.7 ms against 7.4
                 // in cost order.
                 if (rows) {
-                    std::vector<double> cost(nw, 0.0);
-                    parallel_for(nw, [&](size_t i) {
-                        const int kb = nprim(packed[i]);
-                        for (int j = 0; j < packed[2 * nw + i]; ++j) cost[i] += 1.0 + (double)kb * nprim(kets[packed[nw + i] + j]);
-                    }, 512);
                     std::vector<int> o(nw), q(4 * nw);
                     std::iota(o.begin(), o.end(), 0);
-                    std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return cost[x] > cost[y]; });
+                    std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return wsteps[x] > wsteps[y]; });
                     for (int k = 0; k < 4; ++k)
                         for (size_t i = 0; i < nw; ++i) q[k * nw + i] = packed[k * nw + o[i]];
                     packed.swap(q);
-                } else {
-                    // counting sort by the steps' binary exponent
-                    std::vector<unsigned char> key(w.nseg);
-                    std::array<int, 257> at{};
-                    for (int i = 0; i < w.nseg; ++i) {
-                        float x = 0.f;
-                        for (int u = seg[i]; u < seg[i + 1]; ++u) x += wsteps[u];
-                        ++at[1 + (key[i] = (unsigned char)(255 - std::min(255, std::max(0, std::ilogb(x)))))];
-                    }
-                    std::partial_sum(at.begin(), at.end(), at.begin());
-                    std::vector<int> q(2 * (size_t)w.nseg);
-                    for (int i = 0; i < w.nseg; ++i) {
-                        const size_t n = at[key[i]]++;
-                        q[2 * n] = seg[i];
-                        q[2 * n + 1] = seg[i + 1];
-                    }
-                    seg.swap(q);
                 }
                 int rc;
                 if ((rc = dev_upload(&w.d_wave, packed, c->stream)) != PK_OK) return rc;
