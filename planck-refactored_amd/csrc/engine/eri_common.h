@@ -49,6 +49,12 @@ struct PrimDev {
     double pa[3];
 };
 
+// Element (r, c) of a matrix of nb columns, in 64 bits: r nb passes 2^31 from 46341
+// functions on, and a molecule may have 2^20.
+__host__ __device__ constexpr size_t elem(int r, int nb, int c) {
+    return (size_t)(unsigned)r * (unsigned)nb + (unsigned)c;
+}
+
 // ---------------------------------------------------------------- Cartesian order
 // Components of a shell of angular momentum l in the reference order
 // (src/basis/basis.cpp:20-37): lx descending, then ly descending.

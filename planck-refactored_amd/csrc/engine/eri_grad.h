@@ -247,18 +247,18 @@ __global__ __launch_bounds__(64) void k_grad(GradArgs a) {
             const int s = e / PE, t = e - s * PE;
             const int c0 = __shfl(cf0, s * RN, 64), d0 = __shfl(df0, s * RN, 64);
             const double *M;
-            unsigned off;
+            size_t off;
             if (t < 2 * NCD) {
                 const int j = t < NCD ? t : t - NCD;
                 M = t < NCD ? a.Q : a.Pj;
-                off = (unsigned)((c0 + j / ND) * nb + d0 + j % ND);
+                off = elem(c0 + j / ND, nb, d0 + j % ND);
             } else {
                 int x = t - 2 * NCD;
                 const bool second = NK == 2 && x >= S::NX;
                 if (second) x -= S::NX;
                 M = second ? a.Pk2 : a.Pk1;
                 const int r = x / NCX, col = x - r * NCX;
-                off = (unsigned)((r < NA ? bf0 + r : bf1 + r - NA) * nb + (col < NC ? c0 + col : d0 + col - NC));
+                off = elem(r < NA ? bf0 + r : bf1 + r - NA, nb, col < NC ? c0 + col : d0 + col - NC);
             }
             const double x = M[off];
             if (64 * (i + 1) <= QW * PE || lane + 64 * i < QW * PE) G[lane + 64 * i] = x;

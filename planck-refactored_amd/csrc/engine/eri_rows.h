@@ -391,18 +391,18 @@ __device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, 
                 const int s = e / PE, t = e - s * PE;
                 const int c0 = at_slot(cf0, s), d0 = at_slot(df0, s);
                 const double *M;
-                unsigned off;
+                size_t off;
                 if (t < 2 * NCD) {
                     const int j = t < NCD ? t : t - NCD;
                     M = t < NCD ? Qm : P;
-                    off = (unsigned)((c0 + j / ND) * nb + d0 + j % ND);
+                    off = elem(c0 + j / ND, nb, d0 + j % ND);
                 } else {
                     int x = t - 2 * NCD;
                     const bool second = NK == 2 && x >= S::NX;
                     if (second) x -= S::NX;
                     M = second ? KD[1] : KD[0];
                     const int r = x / NCX, col = x - r * NCX;
-                    off = (unsigned)((r < NA ? bf0 + r : bf1 + r - NA) * nb + (col < NC ? c0 + col : d0 + col - NC));
+                    off = elem(r < NA ? bf0 + r : bf1 + r - NA, nb, col < NC ? c0 + col : d0 + col - NC);
                 }
                 st[i] = M[off];
             });
