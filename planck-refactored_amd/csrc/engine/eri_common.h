@@ -55,6 +55,12 @@ __host__ __device__ constexpr size_t elem(int r, int nb, int c) {
     return (size_t)(unsigned)r * (unsigned)nb + (unsigned)c;
 }
 
+// Position g + s in a ket list, the last one before kend beyond it (groups are looked
+// up ahead of the end).  Unsigned: a list may end at 2^31 - 1.
+__host__ __device__ constexpr unsigned ket_pos(unsigned g, unsigned s, unsigned kend) {
+    return g + s < kend ? g + s : kend - 1;
+}
+
 // ---------------------------------------------------------------- Cartesian order
 // Components of a shell of angular momentum l in the reference order
 // (src/basis/basis.cpp:20-37): lx descending, then ly descending.

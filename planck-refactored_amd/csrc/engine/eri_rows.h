@@ -146,8 +146,8 @@ __device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, 
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwg = (int)(blockDim.x >> 6);
     const int bra = uload(a.wave_bra + blk);
-    const int kbeg = uload(a.wave_start + blk);
-    const int kend = kbeg + uload(a.wave_count + blk);
+    const unsigned kbeg = uload(a.wave_start + blk);
+    const unsigned kend = kbeg + uload(a.wave_count + blk);
     const int mol = uload(a.wave_mol + blk);
     const long long moff = uload(a.mol_off + mol);
     const int nb = uload(a.mol_nb + mol);
@@ -232,8 +232,8 @@ __device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, 
     // groups of a wave: chunks of a.chunk groups dealt to the waves in turn (kets
     // with the same first shell are neighbours, and their cost falls along the list)
     int left = a.chunk;  // groups of the current chunk after the one that next() left
-    int g0 = kbeg + wid * a.chunk * QW;
-    auto next = [&](int g) {
+    unsigned g0 = kbeg + wid * a.chunk * QW;
+    auto next = [&](unsigned g) {
         if (--left > 0) return g + QW;
         left = a.chunk;
         return g + QW + (nwg - 1) * a.chunk * QW;
@@ -242,11 +242,11 @@ __device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, 
     // ---- software pipeline over the groups: the ket indices are loaded two
     // groups ahead, the pair fields one group ahead, the first ket primitive and
     // the coefficients of its roots before the digestion of the previous group
-    auto slot_ket = [&](int g, int s) { return a.kets[min(g + s, kend - 1)]; };
+    auto slot_ket = [&](unsigned g, int s) { return a.kets[ket_pos(g, s, kend)]; };
     int ida = 0, idb[RPL];                      // kets of the next group (phase A slot, rows)
     int n_qoff, n_nq, n_c0[RPL], n_d0[RPL], n_diag[RPL];
     double n_qmin[RPL], n_cd[RPL][3];
-    auto load_fields = [&](int g) {             // from ida, idb of group g
+    auto load_fields = [&](unsigned g) {             // from ida, idb of group g
         const PairDev *pk = a.pairs + ida;
         const bool on = live_a && g + sa < kend;
         n_nq = on ? pk->nprim : 0;
@@ -261,7 +261,7 @@ __device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, 
             sfor<0, 3>([&](auto q_) { n_cd[k][PK_CI(q_)] = pr->ab[PK_CI(q_)]; });
         });
     };
-    auto load_ids = [&](int g) {
+    auto load_ids = [&](unsigned g) {
         ida = slot_ket(g, live_a ? sa : 0);
         sfor<0, RPL>([&](auto k_) { idb[PK_CI(k_)] = slot_ket(g, sb[PK_CI(k_)]); });
     };
@@ -295,7 +295,7 @@ __device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, 
         for (int j = 0; j <= PK_RYS_DEG; ++j) cc[j] = c[j];
     };
     bool more = false;  // primitives left in the group
-    int g1 = next(g0);
+    unsigned g1 = next(g0);
     if (g0 < kend) {
         load_ids(g0);
         load_fields(g0);
@@ -407,7 +407,7 @@ __device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, 
                 st[i] = M[off];
             });
         }
-        const int g2 = next(g1);
+        const unsigned g2 = next(g1);
         load_fields(g1);
         load_ids(g2);
 

@@ -21,3 +21,12 @@ def test_matrix_elements(tmp_path):
              ((1 << 20) - 1, 1 << 20, (1 << 20) - 1)]
     got = _run(tmp_path, "".join('std::printf("%%zu\\n", pk::elem(%d, %d, %d));\n' % c for c in cases))
     assert got == [r * nb + c for r, nb, c in cases]
+
+
+def test_ket_positions_at_the_end_of_a_full_list(tmp_path):
+    """A wave looks two groups ahead: past the end of the list by up to the turns of
+    four waves of eight groups of 21 kets."""
+    end = (1 << 31) - 1
+    cases = [(0, 0, 1), (5, 3, 9), (5, 3, 8), (end - 1, 0, end), (end - 1, 20, end), (end + 2 * 4 * 8 * 21, 20, end)]
+    got = _run(tmp_path, "".join('std::printf("%%u\\n", pk::ket_pos(%du, %du, %du));\n' % c for c in cases))
+    assert got == [min(g + s, e - 1) for g, s, e in cases]
