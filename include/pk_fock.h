@@ -172,10 +172,14 @@ int pk_eri_gradient(pk_ctx *ctx, const double *Pj, const double *Pk1, const doub
                     int memkind);
 
 /* Per-class device timing (HIP events around each class's kernels on the
- * context stream).  Disabled by default; enabling resets the counters. */
+ * context stream).  Disabled by default; enabling resets the counters.  While
+ * it is enabled the classes run one at a time in kernels of their own, also in
+ * builds that otherwise run them side by side or in one launch: the times are
+ * those of the class kernels, and do not add up to the time of such a build. */
 typedef struct pk_class_stats {
     int32_t la, lb, lc, ld;       /* angular class of the kernels */
-    int32_t kernels;              /* kernels per build (ket-component chunks) */
+    int32_t kernels;              /* kernels per build (ket-component chunks); 1 for a class that
+                                     shares the one launch of a short build */
     int64_t quartets;
     int64_t primitive_quartets;
     double model_flops;           /* flop model v1 of one build of this class */

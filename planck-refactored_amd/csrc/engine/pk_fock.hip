@@ -1227,8 +1227,12 @@ int launch_small(pk_ctx *c, const BuildBufs &sb, int &nl) {
         ++nl;
     }
     int rc;
-    for (ClassWork &w : c->work)
-        if (!small_covers(w) && (rc = launch_list(c, w, sb, false, c->stream, nl)) != PK_OK) return rc;
+    for (ClassWork &w : c->work) {
+        if (small_covers(w))
+            w.kernels = 1, w.block_run = 64;  // the launch it shares
+        else if ((rc = launch_list(c, w, sb, false, c->stream, nl)) != PK_OK)
+            return rc;
+    }
     return PK_OK;
 }
 

@@ -100,3 +100,13 @@ def test_list_eris_match_oracle(mol, basis, kernels):
     _check_kernels(eng, kernels)
     print("%s/%s %s: max|dERI| %.2e" % (mol, basis, kernels, worst))
     assert worst < 1e-11
+
+
+def test_class_statistics_of_a_short_build():
+    """Every class reports its kernels and their shape, also where it shares a launch."""
+    for basis in ("sto-3g", "cc-pvtz"):
+        eng = FockEngine(Molecule(*water(), basis).shells(), "os", 1e-10)
+        eng.jk(_density(eng.nbasis, 4))
+        cls = eng.class_stats()
+        assert eng.stats()["kernel_launches"] < len(cls)
+        assert all(c["kernels"] >= 1 and c["block"] in (64, 128, 256) for c in cls)
