@@ -1189,6 +1189,29 @@ int ensure_side(pk_ctx *c) {
     return PK_OK;
 }
 
+// Side queues of the work at hand: q[0] is the context stream, the others wait for
+// what it holds so far.
+int fork_side(pk_ctx *c, hipStream_t (&q)[kSideQueues + 1]) {
+    q[0] = c->stream;
+    PK_HIP(hipEventRecord(c->fork_ev, c->stream));
+    for (int i = 0; i < kSideQueues; ++i) {
+        q[i + 1] = c->side[i];
+        PK_HIP(hipStreamWaitEvent(c->side[i], c->fork_ev, 0));
+    }
+    return PK_OK;
+}
+
+// The context stream waits for the side queues.  Called after a failed launch as well
+// (status rc, returned): kernels already on them still use the context's buffers.
+int join_side(pk_ctx *c, int rc) {
+    for (int i = 0; i < kSideQueues; ++i) {
+        hipError_t e = hipEventRecord(c->join_ev[i], c->side[i]);
+        if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, c->join_ev[i], 0);
+        if (e != hipSuccess && rc == PK_OK) rc = fail(PK_ERR_HIP, std::string("side queue join: ") + hipGetErrorString(e));
+    }
+    return rc;
+}
+
 // kernel arguments of a build, without those of a list
 pk::JKArgs build_args(const pk_ctx *c, const BuildBufs &sb) {
     pk::JKArgs a{};
@@ -1245,12 +1268,8 @@ int launch_classes(pk_ctx *c, const BuildBufs &sb, bool events, int &nl) {
     // least cost so far, so that the small classes fill the tails of the
     // large ones.  All lists add into the same accumulators with atomics.
     if (!events && c->side_ok && !c->side_off && c->st.quartets >= kSideMinQuartets && c->work.size() > 1) {
-        PK_HIP(hipEventRecord(c->fork_ev, s));
-        hipStream_t q[kSideQueues + 1] = {s};
-        for (int i = 0; i < kSideQueues; ++i) {
-            q[i + 1] = c->side[i];
-            PK_HIP(hipStreamWaitEvent(c->side[i], c->fork_ev, 0));
-        }
+        hipStream_t q[kSideQueues + 1];
+        if ((rc = fork_side(c, q)) != PK_OK) return rc;
         std::vector<size_t> order(c->work.size());
         for (size_t i = 0; i < order.size(); ++i) order[i] = i;
         // cost of a list: its measured time when the context has one (the first
@@ -1270,13 +1289,9 @@ int launch_classes(pk_ctx *c, const BuildBufs &sb, bool events, int &nl) {
             for (int j = 1; j <= kSideQueues; ++j)
                 if (load[j] < load[k]) k = j;
             load[k] += cost[i];
-            if ((rc = launch_list(c, c->work[i], sb, false, q[k], nl)) != PK_OK) return rc;
+            if ((rc = launch_list(c, c->work[i], sb, false, q[k], nl)) != PK_OK) break;
         }
-        for (int i = 0; i < kSideQueues; ++i) {
-            PK_HIP(hipEventRecord(c->join_ev[i], c->side[i]));
-            PK_HIP(hipStreamWaitEvent(s, c->join_ev[i], 0));
-        }
-        return PK_OK;
+        return join_side(c, rc);
     }
     for (ClassWork &w : c->work)
         if ((rc = launch_list(c, w, sb, events, s, nl)) != PK_OK) return rc;
@@ -2159,16 +2174,12 @@ int pk_eri_gradient(pk_ctx *c, const double *Pj, const double *Pk1, const double
     hipStream_t q[kSideQueues + 1] = {s};
     int nq = 1;
     if (!c->side_off && c->gwork.size() > 1) {
-        if ((rc = ensure_side(c)) != PK_OK) return rc;
-        PK_HIP(hipEventRecord(c->fork_ev, s));
-        for (int i = 0; i < kSideQueues; ++i) {
-            q[nq++] = c->side[i];
-            PK_HIP(hipStreamWaitEvent(c->side[i], c->fork_ev, 0));
-        }
+        if ((rc = ensure_side(c)) != PK_OK || (rc = fork_side(c, q)) != PK_OK) return rc;
+        nq = kSideQueues + 1;
     }
     double load[kSideQueues + 1] = {};
     const int nk = Pk2 ? 2 : 1;
-    for (const GradWork &w : c->gwork) {
+    auto launch = [&](const GradWork &w, hipStream_t on) -> int {
         const pk::GradEntry &e = grad_table()[w.cls];
         pk::GradArgs a{};
         a.item_bra = w.d_items;
@@ -2197,17 +2208,19 @@ int pk_eri_gradient(pk_ctx *c, const double *Pj, const double *Pk1, const double
             PK_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax));
             done.store(1);
         }
+        void *args[] = {&a};
+        PK_HIP(hipLaunchKernel(k, dim3(w.nitems, e.rc), dim3(64), args, e.lds[nk - 1], on));
+        return PK_OK;
+    };
+    for (const GradWork &w : c->gwork) {
         int j = 0;
         for (int i = 1; i < nq; ++i)
             if (load[i] < load[j]) j = i;
         load[j] += w.cost;
-        void *args[] = {&a};
-        PK_HIP(hipLaunchKernel(k, dim3(w.nitems, e.rc), dim3(64), args, e.lds[nk - 1], q[j]));
+        if ((rc = launch(w, q[j])) != PK_OK) break;
     }
-    for (int i = 1; i < nq; ++i) {
-        PK_HIP(hipEventRecord(c->join_ev[i - 1], q[i]));
-        PK_HIP(hipStreamWaitEvent(s, c->join_ev[i - 1], 0));
-    }
+    if (nq > 1) rc = join_side(c, rc);
+    if (rc != PK_OK) return rc;
     PK_HIP(hipGetLastError());
     const size_t gb = 3 * (size_t)c->ns * sizeof(double);
     PK_HIP(hipMemcpyAsync(grad, c->d_gsh, gb, memkind == PK_MEM_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, s));
