@@ -28,7 +28,7 @@
 //   registers from the densities of the quartet.
 // Work per primitive quartet, root, row and f: six products and six FMAs, nine
 // rows of LDS: bound by LDS and VALU alike; small molecules by the longest chain
-// of primitives.  n-C3H8 / cc-pVDZ (85 functions) 4.1 ms per gradient, 11.4 ms
+// of primitives.  n-C3H8 / cc-pVDZ (85 functions) 3.8 ms per gradient, 11.4 ms
 // without cutting the bra's primitives; 1213 ms with one quartet per wave, every
 // factor and component through LDS and a serial chain of up to 6561 primitive
 // quartets.

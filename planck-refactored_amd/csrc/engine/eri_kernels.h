@@ -125,12 +125,13 @@ __device__ __forceinline__ void os_values(const PairDev &pb, const PairDev &pk, 
 }
 
 // Classes whose per-lane kernel runs in segment mode (LDS exchange rows, see
-// k_jk).  Measured per class on n-C10H22 / cc-pVTZ (segment mode / plain): kets
-// with a p or d second shell 0.26-0.83 (the Rys classes (30|22) 0.26, (30|21) 0.31,
-// (21|11) 0.43); kets (ps) and (ss) 0.60-0.83 ((ps|ps) 5.5 -> 3.9 ms, (pp|ss) 2.7 ->
-// 2.0 ms) with the most expensive segments first; but (00|00) 1.51, (10|00) 1.00
-// (n-C20H42 / cc-pVDZ 1.16), kets (ds) 1.16-1.30 except (20|20) 0.86, kets (fs)
-// 1.05-2.02, and the (ff| bras (20 exchange rows, few kets per bra) 1.10-2.02.
+// k_jk).  Measured per class on n-C10H22 / cc-pVTZ (segment mode / plain, the most
+// expensive segments first): (ds|pp) 0.48, the one per-lane class whose kets have a p
+// second shell; kets (ps) 0.56-0.93 ((ds|ps) 6.7 -> 4.3 ms, (dp|ps) 7.9 -> 6.6, (fd|ps)
+// 4.7 -> 4.4); kets (ss) 0.45-0.75 ((ds|ss) 4.9 -> 3.1 ms, (pp|ss) 2.9 -> 1.7); (ds|ds)
+// 0.61; but (ss|ss) 1.35, (ps|ss) 1.09 (n-C20H42 / cc-pVDZ 1.41 and 1.19), the other
+// kets (ds) 1.00-1.12, and the (ff| bras (20 exchange rows, few kets per bra) 1.22
+// for (ps) kets, 1.57 for (ss).
 constexpr bool seg_class(int la, int lb, int lc, int ld) {
     if (la == 3 && lb == 3) return false;
     if (ld >= 1) return true;

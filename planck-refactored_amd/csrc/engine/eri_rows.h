@@ -240,8 +240,9 @@ __device__ __forceinline__ void rows_run(const JKArgs &a, int blk, int chunk_y, 
     };
 
     // ---- software pipeline over the groups: the ket indices are loaded two
-    // groups ahead, the pair fields one group ahead, the first ket primitive and
-    // the coefficients of its roots before the digestion of the previous group
+    // groups ahead, the pair fields one group ahead (ket primitives and the
+    // coefficients of their roots where they are used: loading them one primitive
+    // quartet ahead changed nothing, the LDS pipe and the vector unit set the time)
     auto slot_ket = [&](unsigned g, int s) { return a.kets[ket_pos(g, s, kend)]; };
     int ida = 0, idb[RPL];                      // kets of the next group (phase A slot, rows)
     int n_qoff, n_nq, n_c0[RPL], n_d0[RPL], n_diag[RPL];

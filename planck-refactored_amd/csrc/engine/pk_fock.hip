@@ -92,7 +92,7 @@ constexpr double kCutWaves = 8192.0, kCutSteps = 32.0;
 // takes the row kernel (fewer than the lanes of two waves per SIMD)
 constexpr size_t kRowsFew = 2 * 64 * 4 * 256;
 // A build whose lists hold at most kSmallWaves waves and work items in all is
-// short: its lists go out in one launch (k_small).  H2O / 6-31G* 0.76 -> 0.07 ms,
+// short: its lists go out in one launch (k_small).  H2O / 6-31G* 0.76 -> 0.08 ms,
 // three waters 1.47 -> 0.32 ms, H2O / cc-pVTZ 4.3 -> 0.72 ms; above it the lists
 // win by themselves (n-C2H6 / cc-pVTZ, 60 thousand waves, 2.6 ms against 4.9 ms).
 constexpr int64_t kSmallWaves = 32768;
@@ -1334,7 +1334,11 @@ int launch_list(pk_ctx *c, ClassWork &w, const BuildBufs &sb, bool events, hipSt
             const size_t wave_bytes = r.wave_bytes[rk - 1];
             const void *k = uhf ? r.k2 : r.k1;
             // exchange rows of the kets' second shells in LDS, beside at least one
-            // wave
+            // wave.  Even where they leave room for few waves they win as a whole:
+            // 40 waters 6 Angstrom apart / cc-pVTZ (2600 functions, rows of up to 134 KB)
+            // 319 ms against 462 without rows, (fd|dp) 3.4 / 7.9, (fd|pp) 3.7 / 11.5;
+            // only lists of few kets per row column lose, (ff|fp) 2.2 / 1.1, (fd|fd)
+            // 1.0 / 0.5, (ff|ff) 0.4 / 0.2, (ff|fs) 1.5 / 1.2, (fs|fs) 2.4 / 2.1.
             const size_t jrow = (size_t)pk::ncart(f.la) * pk::ncart(f.lb) * sizeof(double);
             size_t krow = (size_t)rk * (pk::ncart(f.la) + pk::ncart(f.lb)) * w.kcols * sizeof(double) + jrow;
             a.segmode = c->seg_on && krow + wave_bytes <= kLdsMax;
